@@ -46,14 +46,21 @@ def make_fields(ops_s, shift, Lv, seed=2024):
     return 3.0 * S0 + nA, -3.0 * S0 + nB
 
 
-def stage_bytes(plan, e):
+def line_chain(stages):
+    """Whether the profiled steps ran path QS's line-matrix kernels: one kernel
+    per step and no transforms of planes."""
+    return "p51_unfold_fold" in stages and not ({"p2_fft_yz", "p2q_plane_pair"} & set(stages))
+
+
+def stage_bytes(plan, e, lines=False):
     """Algorithmic HBM bytes per launch of each stage (tables excluded):
     each distinct input array read once, each output written once; fields of
-    e bytes, interaction factors E of 8 bytes in both precisions."""
+    e bytes, interaction factors E of 8 bytes in both precisions; channels
+    complex, or real for the line-matrix kernels (`lines`)."""
     B = plan.batch
     eE = 8
     M3 = int(np.prod(plan.M))
-    chan = plan.n_ch * int(np.prod(plan.H)) * 2 * e
+    chan = plan.n_ch * int(np.prod(plan.H)) * (1 if lines else 2) * e
     spec = plan.n_spec * 2 * e
     rep = plan.n_rep * 2 * e
     qr = plan.path == 5  # orbit-reduced Q chain
@@ -75,12 +82,12 @@ def stage_bytes(plan, e):
     }
 
 
-def launch_bytes(plan, e, stage, steps_per_launch):
+def launch_bytes(plan, e, stage, steps_per_launch, lines=False):
     """Algorithmic bytes of one launch of `stage` (the persistent sweep moves
     one Strang step's bytes per field per contour step)."""
     if stage == "sweep":
         return steps_per_launch * plan.batch * step_bytes(plan, e)
-    return stage_bytes(plan, e)[stage]
+    return stage_bytes(plan, e, lines)[stage]
 
 
 def step_bytes(plan, e):
@@ -149,11 +156,11 @@ STRATEGY_PATH = {"m7_chain": 0, "m7_persistent": 0, "qr_chain": 5, "qs_chain": 6
 TRAFFIC_RECORD = {0: "m7_chain", 5: "qr_chain", 6: "qs_chain"}
 
 
-def profiled_traffic(strategy, stage_name, prec_name, axis=False):
+def profiled_traffic(strategy, stage_name, prec_name, lines=False):
     """HBM bytes per launch of a chain kernel at this workload (2 fields per
     launch), from the FETCH_SIZE / WRITE_SIZE profiler runs recorded under
     profiles/ for the pipeline path of that launch strategy (each counter
-    scaled by what it reads for a plain 64 MiB copy), the per-axis chain's
+    scaled by what it reads for a plain 64 MiB copy), the line-matrix
     kernels under their own keys; None when no such record exists."""
     name = TRAFFIC_RECORD.get(STRATEGY_PATH.get(strategy))
     if name is None:
@@ -161,7 +168,7 @@ def profiled_traffic(strategy, stage_name, prec_name, axis=False):
     path = os.path.join(ROOT, "profiles", f"hbm_traffic_im3m128_{name}.json")
     try:
         with open(path) as fh:
-            rec = json.load(fh)["kernels"].get(f"{stage_name}/{prec_name}" + ("/axis" if axis else ""))
+            rec = json.load(fh)["kernels"].get(f"{stage_name}/{prec_name}" + ("/lines" if lines else ""))
     except (OSError, ValueError, KeyError):
         return None
     return None if rec is None else float(rec["bytes"])
@@ -373,7 +380,7 @@ def batched_fields(cf, torch, ops_s, wA, prec, e, batch, steps, path, options=No
     dom = dominant_stage(stages)
     E_ptrs = (C.c_void_p * batch)(*[E.data_ptr() + b * M3 * 8 for b in range(batch)])
     avg = live_launch_ms(plan, dom, q.data_ptr(), E_ptrs, s)
-    nb = stage_bytes(plan, e)[dom]
+    nb = stage_bytes(plan, e, line_chain(stages))[dom]
     return {"batch": batch, "value": batch * steps / el, "unit": "diffusion steps/s",
             "ms_per_step": el / steps * 1e3, "dominant_kernel": dom, "avg_launch_ms": avg,
             "achieved_GBs": nb / (avg * 1e-3) / 1e9, "frac": nb / (avg * 1e-3) / 1e9 / HBM_PEAK_GBS}
@@ -721,7 +728,8 @@ def main():
             del scratch
         else:  # persistent sweep: one event pair around each cooperative launch
             avg_ms = stages[dom][0] / stages[dom][1]
-        nb = launch_bytes(sw.plan, e, dom, NS)
+        lines = line_chain(stages)
+        nb = launch_bytes(sw.plan, e, dom, NS, lines)
         achieved = nb / (avg_ms * 1e-3) / 1e9
         # every per-step chain kernel beside the dominant one, timed the same way
         chain = {}
@@ -731,13 +739,13 @@ def main():
             scratch = sw.q.clone()
             ms = avg_ms if st == dom else live_launch_ms(sw.plan, st, scratch.data_ptr(), sw._E1, sw.stream())
             del scratch
-            b = launch_bytes(sw.plan, e, st, NS)
+            b = launch_bytes(sw.plan, e, st, NS, lines)
             chain[st] = {"avg_launch_ms": ms, "bytes_per_launch": b, "achieved": b / (ms * 1e-3) / 1e9,
                          "frac": b / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS}
         res[name] = dict(el=el, med=med, Qq=Qq, Qd=Qd, q=qfields, stages=stages, dom=dom, avg_ms=avg_ms,
                          achieved=achieved, plan=sw.plan, sbytes=nb, chain=chain,
                          step_bytes=step_bytes(sw.plan, e),
-                         axis=bool(sw.plan.options.get(cf._lib.OPT_AXIS_SPLIT)),
+                         lines=lines,
                          options={k: v for k, v in sw.plan.options.items()
                                   if k in (cf._lib.OPT_AXIS_SPLIT, cf._lib.OPT_FFT_LANES,
                                            cf._lib.OPT_PAIR_THREADS)})
@@ -818,7 +826,7 @@ def main():
                                  "(2 Ns diffusion steps)"},
         "roofline": {"bound": "hbm", "kernel": r64["dom"], "achieved": r64["achieved"],
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": r64["achieved"] / HBM_PEAK_GBS,
-                     "traffic": profiled_traffic(variants["fp64"]["used"], r64["dom"], "fp64", r64["axis"]),
+                     "traffic": profiled_traffic(variants["fp64"]["used"], r64["dom"], "fp64", r64["lines"]),
                      "bytes_per_launch": r64["sbytes"],
                      "avg_launch_ms": r64["avg_ms"], "chain_kernels": r64["chain"]},
         "mixed": {"value": mixed_value, "dtype": "f32 data/FFT/propagator, f64 tables+reductions",

@@ -22,7 +22,7 @@ FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 
-SOURCES = [os.path.join(CSRC, f) for f in ("cfft_hip.hip", "blocks.hip", "scft.hip", "mlp.hip", "dense.hip",
+SOURCES = [os.path.join(CSRC, f) for f in ("cfft_hip.hip", "lines.hip", "blocks.hip", "scft.hip", "mlp.hip", "dense.hip",
                                             "ensemble.hip", "p3c.hip", "plan.cpp")]
 
 

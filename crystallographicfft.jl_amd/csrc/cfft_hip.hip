@@ -19,6 +19,7 @@
 #include "kernels.hpp"
 #include "pipeline.hpp"
 #include "ensemble.hpp"
+#include "lines.hpp"
 #include "plan.hpp"
 #include "common.hpp"
 
@@ -46,6 +47,8 @@ struct cfft_plan {
   long n_rep = 0;  // orbit representatives of the alive M-grid (path QR)
   int qs_items = 0;  // plane-pair items per batch entry (path QS)
   int qs_sep = 0;    // path QS: translations separable in the sign pattern
+  int lines_ok = 0;  // path QS: the line-matrix chain applies (a channel's multiply factors per axis)
+  int axv[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // its matrix variants (PipeP::axv)
   size_t esz = 8;  // element size of the plan's real type
   hipStream_t stream = nullptr;
   // device tables
@@ -54,6 +57,7 @@ struct cfft_plan {
   DevBuf d_f0, d_ch, d_ch2, d_F, d_E, d_u;
   DevBuf d_qmap, d_grep;  // path QR: element -> (rep, phase); rep values
   DevBuf d_qsep;          // path QS: axis factors F[d][s][q]
+  DevBuf d_lines;         // path QS: line matrices (lines.hpp)
   DevBuf d_symops;        // ops that keep the subgrid, acting on it (12 int32 each)
   int n_sym = 0;
   std::vector<int32_t> fmap_host;
@@ -134,6 +138,11 @@ void upload_bytes(DevBuf& buf, const void* src, size_t n) {
   if (n) hip_check(hipMemcpy(buf.p, src, n, hipMemcpyHostToDevice), "upload");
 }
 
+// Path QS with a channel's multiply separable per axis: the plan's steps run
+// the line-matrix chain, unless a lane split of the plane-pair transforms was
+// asked for (CFFT_OPT_FFT_LANES, which selects the plane-pair kernels).
+bool use_lines(const cfft_plan* p) { return is_qs(p) && p->lines_ok && !p->lanes; }
+
 // Path QS axis factors F[d][s][q], q < M_d, s = sign pattern of the
 // representative op (bit i: R_ii = -1):
 //   F_d[s][q] = sum_{a in {0,1}} K_d(q + M_d a) exp(-2 pi i (q + M_d a) t_{s,d} / N_d),
@@ -146,6 +155,107 @@ bool orthogonal_cell(const double* A) {  // column-major 3 x 3
     for (int j = 0; j < 3; ++j)
       if (i != j && A[i + 3 * j] != 0.0) return false;
   return true;
+}
+
+// Whether channel c's multiply factors per axis, and the matrices if so.
+// Every op's translation component must be the one of the pure flip of its
+// axis (0 unflipped) plus 0 or half the grid: e^{-2 pi i h (N/2)/N} = (-1)^h
+// is the sign (-1)^(o tau) on channel parity o, and the op's sign on a
+// channel, sigma_c(s) = (-1)^(sum_d o_d tau_d(s)), must be the product of its
+// single flips' (mirrors with the magic shift: tau = 0 throughout; the
+// half-cell glides of Ia-3d: sigma separable on the I-centred channels;
+// quarter-cell glides, Fddd and Fd-3m: no).
+void build_lines(cfft_plan* p, const int (&tsel)[8][3]) {
+  p->lines_ok = 0;
+  if (!line_len_ok(p->H[0])) return;
+  int tau[8][3];
+  for (int s = 0; s < 8; ++s)
+    for (int d = 0; d < 3; ++d) {
+      const int ref = ((s >> d) & 1) ? tsel[1 << d][d] : 0;
+      const int df = (((tsel[s][d] - ref) % p->N[d]) + p->N[d]) % p->N[d];
+      if (df != 0 && 2 * df != p->N[d]) return;
+      tau[s][d] = df ? 1 : 0;
+    }
+  for (int c = 0; c < p->n_ch; ++c) {
+    auto sigma = [&](int s) {
+      int v = 0;
+      for (int d = 0; d < 3; ++d) v ^= p->offs[c][d] & tau[s][d];
+      return v;
+    };
+    for (int s = 0; s < 8; ++s) {
+      int v = 0;
+      for (int d = 0; d < 3; ++d)
+        if ((s >> d) & 1) v ^= sigma(1 << d);
+      if (sigma(s) != v) return;
+    }
+    p->axv[c] = 0;
+    for (int d = 0; d < 3; ++d) p->axv[c] |= (p->offs[c][d] | (sigma(1 << d) << 1)) << (2 * d);
+  }
+  // Sums in extended precision; the entries of a row are rounded to double
+  // largest first, each taking the rounding error of those before it, so a
+  // row keeps its sum (the gain of the k = 0 mode, which acts on every step
+  // alike) to the last bit of its smallest entries.
+  const int H = p->H[0], M = 2 * H, KS = H / 4, VAR = line_variant_len(H);
+  const long double tp = 2.0L * 3.14159265358979323846264338327950288L;
+  std::vector<double> tab((size_t)12 * VAR, 0.0);
+  std::vector<long double> cr(M), ci(M), T(2 * H), W(2 * H), f0(M), f1r(M), f1i(M), row(H);
+  std::vector<int> by(H);
+  for (int j = 0; j < M; ++j) {
+    cr[j] = cosl(tp * j / M);
+    ci[j] = sinl(tp * j / M);
+  }
+  for (int d = 0; d < 3; ++d) {
+    const long double bd = tp / p->lattice[d + 3 * d];
+    for (int q = 0; q < M; ++q) {  // (1/2) sum_a K(q + M a) [e^{-2 pi i (q + M a) t / N}]
+      f0[q] = f1r[q] = f1i[q] = 0.0L;
+      for (int a = 0; a < 2; ++a) {
+        const long h = q + (long)M * a;
+        const long double kv = bd * k_centered((int)h, p->N[d]);
+        const long double kd = 0.5L * expl(-kv * kv * (long double)p->ds);
+        const long double ph = tp * (long double)((((long long)h * tsel[1 << d][d]) % p->N[d])) / p->N[d];
+        f0[q] += kd;
+        f1r[q] += kd * cosl(ph);
+        f1i[q] -= kd * sinl(ph);
+      }
+    }
+    for (int o = 0; o < 2; ++o) {
+      // A[x'][x] = T[x' - x + H] + chi W[x' + x]
+      for (int n = 0; n < 2 * H; ++n) {
+        T[n] = W[n] = 0.0L;
+        for (int k = 0; k < H; ++k) {
+          const int q = 2 * k + o;
+          const int jt = (int)((((long)q * (n - H)) % M + M) % M), jw = (int)(((long)q * n) % M);
+          T[n] += f0[q] * cr[jt] / H;
+          W[n] += (f1r[q] * cr[jw] - f1i[q] * ci[jw]) / H;
+        }
+      }
+      for (int chi = 0; chi < 2; ++chi) {
+        double* v = tab.data() + ((size_t)d * 4 + o + 2 * chi) * VAR;
+        for (int r = 0; r < H; ++r) {
+          for (int x = 0; x < H; ++x) {
+            row[x] = T[r - x + H] + (chi ? -W[r + x] : W[r + x]);
+            by[x] = x;
+          }
+          std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return fabsl(row[a]) > fabsl(row[b]); });
+          long double err = 0.0L;
+          for (int x : by) {
+            const double e = (double)(row[x] + err);
+            err += row[x] - e;
+            // lane and k-step of column x in the two contraction orders (lines.hpp)
+            const int i = d == 0 ? x % KS : x / 4, g = d == 0 ? x / KS : x % 4;
+            v[line_entry(H, r / 16, i, 16 * g + r % 16)] = e;
+          }
+        }
+      }
+    }
+  }
+  if (!p->d_lines.p) {
+    upload_bytes(p->d_lines, tab.data(), tab.size() * sizeof(double));
+  } else {  // same allocation: captured chains keep pointing at it
+    std::lock_guard<std::recursive_mutex> guard(setup_mutex());
+    hip_check(hipMemcpy(p->d_lines.p, tab.data(), p->d_lines.bytes, hipMemcpyHostToDevice), "upload line matrices");
+  }
+  p->lines_ok = 1;
 }
 
 void build_qs_table(cfft_plan* p) {
@@ -204,6 +314,7 @@ void build_qs_table(cfft_plan* p) {
     std::lock_guard<std::recursive_mutex> guard(setup_mutex());
     hip_check(hipMemcpy(p->d_qsep.p, h.data(), p->d_qsep.bytes, hipMemcpyHostToDevice), "upload QS factors");
   }
+  build_lines(p, tsel);
   p->qs_items = 0;
   // orbits of x -> xbar: xbar = (H - x) mod H (offset 0) or H - 1 - x (offset 1)
   for (int c = 0; c < p->n_ch; ++c) p->qs_items += p->offs[c][0] ? (p->H[0] + 1) / 2 : p->H[0] / 2 + 1;
@@ -637,6 +748,7 @@ PipeP pipe_params(cfft_plan* p, const ESel& es) {
   pp.n_rep = p->n_rep;
   pp.qs_items = p->qs_items;
   pp.qs_sep = p->qs_sep;
+  for (int c = 0; c < 8; ++c) pp.axv[c] = p->axv[c];
   return pp;
 }
 
@@ -655,6 +767,7 @@ PipeBufs pipe_bufs(cfft_plan* p, const void* f0_in, void* f0_out, void* F, bool 
   B.grep = p->d_grep.p;
   B.qmap = static_cast<const uint32_t*>(p->d_qmap.p);
   B.qsep = p->d_qsep.p;
+  B.lines = static_cast<const double*>(p->d_lines.p);
   return B;
 }
 
@@ -794,7 +907,21 @@ void launch_qr(cfft_plan* p, const PipeP& pp, const PipeBufs& B, hipStream_t s) 
   launch_check<T>("k_p4r");
 }
 
-// Path QS middle of a step: one kernel per plane pair.
+// Path QS middle of a step: one kernel per plane pair.  A separable plan runs
+// the line-matrix chain instead (use_lines) except at lengths that chain has
+// no kernel for and with a lane split, so the separable multiply is compiled
+// for those; the general multiply gives the same operator.
+template <typename T, typename TW, int L, int NT, int LANES>
+void launch_pair(const PipeP& pp, const PipeBufs& B, unsigned g, hipStream_t s) {
+  if constexpr (LANES != 0 || L < kLineLens[0]) {
+    if (pp.qs_sep) {
+      hipLaunchKernelGGL((k_p2q<T, TW, L, true, NT, LANES>), dim3(g), dim3(NT), 0, s, pp, B);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_p2q<T, TW, L, false, NT, LANES>), dim3(g), dim3(NT), 0, s, pp, B);
+}
+
 template <typename T>
 void launch_p2q(cfft_plan* p, const PipeP& pp, const PipeBufs& B, hipStream_t s) {
   StageTimer st(p, s, CFFT_STAGE_PLANE_Q);
@@ -802,11 +929,8 @@ void launch_p2q(cfft_plan* p, const PipeP& pp, const PipeBufs& B, hipStream_t s)
   bool f32 = false;  // FP32-arithmetic kernels are instantiated for FP32 data only
   if constexpr (std::is_same<T, float>::value) {
     if (fp32_arith(p)) {
-#define CFFT_P2Q(L)                                                                          \
-  case L:                                                                                    \
-    if (pp.qs_sep) hipLaunchKernelGGL((k_p2q<T, float, L, true>), dim3(g), dim3(kQNT), 0, s, pp, B); \
-    else hipLaunchKernelGGL((k_p2q<T, float, L, false>), dim3(g), dim3(kQNT), 0, s, pp, B);          \
-    break;
+#define CFFT_P2Q(L) \
+  case L: launch_pair<T, float, L, kQNT, 0>(pp, B, g, s); break;
       CFFT_LEN_SWITCH(p->H[1], CFFT_P2Q)
 #undef CFFT_P2Q
       f32 = true;
@@ -815,12 +939,11 @@ void launch_p2q(cfft_plan* p, const PipeP& pp, const PipeBufs& B, hipStream_t s)
   if (!f32 && (p->lanes || p->pair_threads)) {
     // a tuned schedule (set_option checked that it is instantiated)
     const int nt = p->pair_threads ? p->pair_threads : kQNT;
-#define CFFT_P2Q_SCHED(L, NT, LN)                                                                  \
-  if (p->H[1] == L && nt == NT && p->lanes == LN) {                                                \
-    if (pp.qs_sep) hipLaunchKernelGGL((k_p2q<T, double, L, true, NT, LN>), dim3(g), dim3(NT), 0, s, pp, B); \
-    else hipLaunchKernelGGL((k_p2q<T, double, L, false, NT, LN>), dim3(g), dim3(NT), 0, s, pp, B);          \
-    launch_check<T>("k_p2q");                                                                      \
-    return;                                                                                        \
+#define CFFT_P2Q_SCHED(L, NT, LN)                       \
+  if (p->H[1] == L && nt == NT && p->lanes == LN) {     \
+    launch_pair<T, double, L, NT, LN>(pp, B, g, s);     \
+    launch_check<T>("k_p2q");                           \
+    return;                                             \
   }
     CFFT_P2Q_SCHED(32, 256, 2) CFFT_P2Q_SCHED(32, 512, 0) CFFT_P2Q_SCHED(32, 512, 2)
     CFFT_P2Q_SCHED(16, 256, 2) CFFT_P2Q_SCHED(16, 512, 0) CFFT_P2Q_SCHED(16, 512, 2)
@@ -829,11 +952,8 @@ void launch_p2q(cfft_plan* p, const PipeP& pp, const PipeBufs& B, hipStream_t s)
     throw Error{CFFT_ERR_UNSUPPORTED, "no plane-pair kernel for this schedule"};
   }
   if (!f32) {
-#define CFFT_P2Q(L)                                                                           \
-  case L:                                                                                     \
-    if (pp.qs_sep) hipLaunchKernelGGL((k_p2q<T, double, L, true>), dim3(g), dim3(kQNT), 0, s, pp, B); \
-    else hipLaunchKernelGGL((k_p2q<T, double, L, false>), dim3(g), dim3(kQNT), 0, s, pp, B);          \
-    break;
+#define CFFT_P2Q(L) \
+  case L: launch_pair<T, double, L, kQNT, 0>(pp, B, g, s); break;
     CFFT_LEN_SWITCH(p->H[1], CFFT_P2Q)
 #undef CFFT_P2Q
   }
@@ -882,67 +1002,25 @@ void launch_p51(cfft_plan* p, const PipeP& pp, const PipeBufs& B, int step, hipS
   launch_check<T>("k_p51");
 }
 
-// The axis-split chain (CFFT_OPT_AXIS_SPLIT): H = 8, 12, 16, 24 or 32, FP64
-// factor and twiddle products in both precisions.
-#define CFFT_AX_SWITCH(len, MACRO) \
-  switch (len) {                   \
-    MACRO(8)                       \
-    MACRO(12)                      \
-    MACRO(16)                      \
-    MACRO(24)                      \
-    MACRO(32)                      \
-    default: throw Error{CFFT_ERR_UNSUPPORTED, "the axis-split chain needs H = 8, 12, 16, 24 or 32"}; \
-  }
-
-template <typename T>
-void launch_p1x(cfft_plan* p, const PipeP& pp, const PipeBufs& B, int step, hipStream_t s) {
+// Line-matrix chain (path QS, use_lines): the first kernel of a chain (E,
+// fold, z-lines into half 0 of the channels), a kernel between two steps, and
+// the last (unfold, E into f0_out).  Kernel n of a chain reads half n of the
+// channels (mod 2) and takes y-lines for even n, z-lines for odd n.
+void launch_lines_first(cfft_plan* p, const PipeP& pp, const PipeBufs& B, int step, hipStream_t s) {
   StageTimer st(p, s, CFFT_STAGE_FOLD);
-  const unsigned g = (unsigned)n_tiles(p, pp);
-#define CFFT_P1X(L) \
-  case L: hipLaunchKernelGGL((k_p1x<T, double, L>), dim3(g), dim3(kNT), 0, s, pp, B, step); break;
-  CFFT_AX_SWITCH(p->H[0], CFFT_P1X)
-#undef CFFT_P1X
-  launch_check<T>("k_p1x");
+  launch_lines(p->prec, p->H[0], p->cent, kLinesOut, pp, B, step, 2, 1, s);
 }
 
-template <typename T>
-void launch_p2x(cfft_plan* p, const PipeP& pp, const PipeBufs& B, hipStream_t s) {
-  StageTimer st(p, s, CFFT_STAGE_PLANE_Q);
-  const unsigned g = (unsigned)n_planes(p);
-#define CFFT_P2X(L)                                                                                  \
-  case L:                                                                                            \
-    hipLaunchKernelGGL((k_p2x<T, double, L>), dim3(g), dim3(L * LineSplit<L>::R1), 0, s, pp, B); \
-    break;
-  CFFT_AX_SWITCH(p->H[1], CFFT_P2X)
-#undef CFFT_P2X
-  launch_check<T>("k_p2x");
-}
-
-template <typename T>
-void launch_p51x(cfft_plan* p, const PipeP& pp, const PipeBufs& B, int step, hipStream_t s) {
+void launch_lines_mid(cfft_plan* p, const PipeP& pp, const PipeBufs& B, int step, int n, hipStream_t s) {
   StageTimer st(p, s, CFFT_STAGE_UNFOLD_FOLD);
-  const unsigned g = (unsigned)n_tiles(p, pp);
-#define CFFT_P51X(L)                                                                                       \
-  case L:                                                                                                  \
-    if (B.f0_out) hipLaunchKernelGGL((k_p51x<T, double, L, true>), dim3(g), dim3(kNT), 0, s, pp, B, step); \
-    else hipLaunchKernelGGL((k_p51x<T, double, L, false>), dim3(g), dim3(kNT), 0, s, pp, B, step);        \
-    break;
-  CFFT_AX_SWITCH(p->H[0], CFFT_P51X)
-#undef CFFT_P51X
-  launch_check<T>("k_p51x");
+  const int mode = kLinesIn | kLinesOut | (B.f0_out ? kLinesStore : 0);
+  launch_lines(p->prec, p->H[0], p->cent, mode, pp, B, step, 1 + (n & 1), n & 1, s);
 }
 
-template <typename T>
-void launch_p5x(cfft_plan* p, const PipeP& pp, const PipeBufs& B, int step, hipStream_t s) {
+void launch_lines_last(cfft_plan* p, const PipeP& pp, const PipeBufs& B, int step, int n, hipStream_t s) {
   StageTimer st(p, s, CFFT_STAGE_UNFOLD);
-  const unsigned g = (unsigned)n_tiles(p, pp);
-#define CFFT_P5X(L) \
-  case L: hipLaunchKernelGGL((k_p5x<T, double, L>), dim3(g), dim3(kNT), 0, s, pp, B, step); break;
-  CFFT_AX_SWITCH(p->H[0], CFFT_P5X)
-#undef CFFT_P5X
-  launch_check<T>("k_p5x");
+  launch_lines(p->prec, p->H[0], p->cent, kLinesIn, pp, B, step, 1 + (n & 1), n & 1, s);
 }
-#undef CFFT_AX_SWITCH
 
 // Work buffers of one diffusion call: channel spectra, the Q-multiplied
 // channels (paths M2Q, M7Q) and the spectral ASU values (paths M2, M7).
@@ -988,10 +1066,9 @@ void run_diffuse(cfft_plan* p, const T* in, T* out_f0, const PipeP& pp, int step
   const Work w = wk ? *wk : own_work(p);
   if (is_qs(p)) {
     PipeBufs B = pipe_bufs(p, in, out_f0, nullptr, false, w.ch);
-    if (p->axis_split) {
-      launch_p1x<T>(p, pp, B, step, s);
-      launch_p2x<T>(p, pp, B, s);
-      launch_p5x<T>(p, pp, B, step, s);
+    if (use_lines(p)) {
+      launch_lines_first(p, pp, B, step, s);
+      launch_lines_last(p, pp, B, step, 0, s);
       return;
     }
     launch_p1<T>(p, pp, B, step, s);
@@ -1183,18 +1260,19 @@ PipeBufs inner_bufs(PipeBufs B, long stride) {
 template <typename T>
 void run_chain(cfft_plan* p, T* q, long stride, const PipeP& pp, int step0, int nsteps, hipStream_t s) {
   cx<T>* F = static_cast<cx<T>*>(p->d_F.p);
-  if (is_qs(p) && p->axis_split) {
-    // per step: the plane kernel (A_y A_z), then the unfold of the step fused
-    // with the fold and A_x of the next
-    launch_p1x<T>(p, pp, pipe_bufs(p, q, nullptr, nullptr, false), step0, s);
+  if (use_lines(p)) {
+    // one kernel per step between the first fold and the last unfold
+    launch_lines_first(p, pp, pipe_bufs(p, q, nullptr, nullptr, false), step0, s);
+    int n = 0;
     for (int i = 0; i < nsteps; ++i) {
       PipeBufs B = pipe_bufs(p, q + (i + 1) * stride, q + (i + 1) * stride, F, false);
-      launch_p2x<T>(p, pp, B, s);
       if (i + 1 < nsteps && p->fuse) {
-        launch_p51x<T>(p, pp, inner_bufs(B, stride), step0 + i, s);
+        launch_lines_mid(p, pp, inner_bufs(B, stride), step0 + i, n, s);
+        ++n;
       } else {
-        launch_p5x<T>(p, pp, B, step0 + i, s);
-        if (i + 1 < nsteps) launch_p1x<T>(p, pp, B, step0 + i + 1, s);
+        launch_lines_last(p, pp, B, step0 + i, n, s);
+        n = 0;
+        if (i + 1 < nsteps) launch_lines_first(p, pp, B, step0 + i + 1, s);
       }
     }
     return;
@@ -1323,13 +1401,13 @@ template <typename T>
 double time_stage(cfft_plan* p, T* q, const ESel& es, int stage, int reps, hipStream_t s) {
   PipeP pp = pipe_params(p, es);
   PipeBufs B = pipe_bufs(p, nullptr, q, p->d_F.p, false);
-  const bool ax = is_qs(p) && p->axis_split;
+  const bool lm = use_lines(p);  // its two kernels: y-lines and z-lines
   auto launch = [&] {
     if (stage == CFFT_STAGE_UNFOLD_FOLD) {
-      if (ax) launch_p51x<T>(p, pp, inner_bufs(B, 0), 0, s);
+      if (lm) launch_lines_mid(p, pp, inner_bufs(B, 0), 0, 0, s);
       else launch_p51<T>(p, pp, inner_bufs(B, 0), 0, s);  // as between two steps of a sweep
     } else if (stage == CFFT_STAGE_PLANE_Q) {
-      if (ax) launch_p2x<T>(p, pp, B, s);
+      if (lm) launch_lines_mid(p, pp, inner_bufs(B, 0), 0, 1, s);
       else launch_p2q<T>(p, pp, B, s);
     } else {
       launch_p2<T>(p, pp, B, s);
@@ -1392,11 +1470,12 @@ EnsPlanInfo ens_plan_info(cfft_plan* p) {
   i.L = p->H[0];
   i.cubic = cubic(p) ? 1 : 0;
   i.batch = p->batch;
-  i.sep = p->qs_sep ? 1 : 0;
+  i.lines = use_lines(p) ? 1 + p->cent : 0;
   i.lanes = p->lanes;
   i.axis_split = p->axis_split;
   i.pair_items = (long)p->qs_items * p->batch;
   i.tile_items = n_tiles(p, pipe_params(p, ESel{}));
+  i.line_items = (long)p->batch * p->H[0] * line_tiles(p->H[0]);
   i.M3 = p->M3;
   return i;
 }

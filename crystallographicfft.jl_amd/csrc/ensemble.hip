@@ -1,10 +1,11 @@
-// Multi-plan history sweeps on the plane-pair Q chain.  The plans of an
-// ensemble fall into classes by channel transform length; per class, one
-// launch per chain stage and contour step takes the plane pairs (or the
-// unfold/fold tiles) of the active fields of every plan of the class from a
-// work list, whatever the plan's grid, space group and batch.  Each class
-// replays its launch sequence from its own hipGraph on its own stream, so
-// the classes run concurrently.  Every work item runs the same phase function, with the same
+// Multi-plan history sweeps of path QS.  The plans of an ensemble fall into
+// classes by channel transform length and chain (the plane-pair chain, or the
+// line-matrix chain by centring, whose workgroups hold one wave per channel);
+// per class, one launch per chain stage and contour step takes the work items
+// of the active fields of every plan of the class from a work list, whatever
+// the plan's grid, space group and batch.  Each class replays its launch
+// sequence from its own hipGraph on its own stream, so the classes run
+// concurrently.  Every work item runs the same phase function, with the same
 // parameters and buffers, as the plan's own sweep (cfft_sweep_hist_dev), so
 // the results are the plan's bit for bit.
 #include <hip/hip_runtime.h>
@@ -30,8 +31,27 @@ __device__ __forceinline__ const EnsSlot& ens_slot(const EnsSlot* S, int k) {
   return *(const EnsSlot*)((ConstSlot*)S + k);
 }
 
+// A kernel of the line-matrix chain over the listed parts (item: (plane of
+// all batch entries) * parts + part), as launched by the plan's own sweep:
+// step -1 folds slice 0, otherwise q(step + 1) goes to its slice.
+template <typename T, int L, int CENT, int MODE>
+__global__ void __launch_bounds__(64 * LineCent<CENT>::NCH) k_lines_ens(const EnsSlot* __restrict__ S, const int* __restrict__ count,
+                                                        const EnsWork* __restrict__ work, int step, int line,
+                                                        int flip) {
+  constexpr int NT = line_tiles(L);
+  __shared__ double lds[LineCent<CENT>::NCH * L * 16];
+  if ((int)blockIdx.x >= *count) return;
+  const EnsWork wk = work[blockIdx.x];
+  const EnsSlot& s = ens_slot(S, wk.slot);
+  PipeBufs B = s.B;
+  B.f0_in = s.q;
+  if (MODE != kLinesOut) B.f0_out = static_cast<T*>(s.q) + (long)(step + 1) * s.stride;
+  const int pl = wk.item / NT;
+  ph_lines<T, L, CENT, MODE>(s.p, B, pl / L, pl % L, wk.item % NT, step, line, flip, lds);
+}
+
 // Plane pairs (FFT y, z, Q multiply, IFFT z, y) of the listed plans.
-template <typename T, int L, bool SEP>
+template <typename T, int L>
 __global__ void __launch_bounds__(kQNT) k_p2q_ens(const EnsSlot* __restrict__ S, const int* __restrict__ count,
                                                   const EnsWork* __restrict__ work) {
   __shared__ cx<T> lds[2 * L * kRow<T, L>];
@@ -39,7 +59,7 @@ __global__ void __launch_bounds__(kQNT) k_p2q_ens(const EnsSlot* __restrict__ S,
   if ((int)blockIdx.x >= *count) return;
   const EnsWork wk = work[blockIdx.x];
   const EnsSlot& s = ens_slot(S, wk.slot);
-  ph_plane_pair_q<T, double, L, kQNT, SEP>(s.p, s.B, wk.item, lds, fq);
+  ph_plane_pair_q<T, double, L, kQNT, false>(s.p, s.B, wk.item, lds, fq);
 }
 
 // Fold + E + FFT x of slice 0 (the first step of a sweep).
@@ -82,11 +102,11 @@ __global__ void __launch_bounds__(kNT) k_p5_ens(const EnsSlot* __restrict__ S, c
   ph_ifftx_unfold<T, double, L>(s.p, B, wk.item, step, lds);
 }
 
-// The work lists of a class: plane pairs of the separable-multiply plans, of
-// the others, and the tiles of all.
-enum { kListSep = 0, kListGen = 1, kListTile = 2, kListsPerClass = 3 };
+// The work lists of a class: plane pairs and tiles, or (line-matrix chain)
+// the second only, its parts of planes.
+enum { kListPair = 0, kListTile = 1, kListsPerClass = 2 };
 
-// Where a class's lists live: entry counts at count[0..2], entries of list t
+// Where a class's lists live: entry counts at count[0..1], entries of list t
 // at work + off[t], at most cap[t] of them (the grid size of its launches).
 struct ClassLists {
   const int* count;
@@ -95,35 +115,53 @@ struct ClassLists {
   unsigned cap[kListsPerClass];
 };
 
+template <typename T, int L, int CENT>
+void capture_lines(const EnsSlot* S, const ClassLists& c, int ns, hipStream_t s) {
+  const int* n = c.count + kListTile;
+  const EnsWork* w = c.work + c.off[kListTile];
+  const dim3 grid(c.cap[kListTile]), block(64 * LineCent<CENT>::NCH);
+  constexpr int kMid = kLinesIn | kLinesOut | kLinesStore;
+  hipLaunchKernelGGL((k_lines_ens<T, L, CENT, kLinesOut>), grid, block, 0, s, S, n, w, 0, 2, 1);
+  for (int i = 0; i + 1 < ns; ++i)
+    hipLaunchKernelGGL((k_lines_ens<T, L, CENT, kMid>), grid, block, 0, s, S, n, w, i, 1 + (i & 1), i & 1);
+  const int i = ns - 1;
+  hipLaunchKernelGGL((k_lines_ens<T, L, CENT, kLinesIn>), grid, block, 0, s, S, n, w, i, 1 + (i & 1), i & 1);
+}
+
 template <typename T, int L>
-void capture_class(const EnsSlot* S, const ClassLists& c, int ns, hipStream_t s) {
-  const int* n_sep = c.count + kListSep;
-  const int* n_gen = c.count + kListGen;
+void capture_class(int lines, const EnsSlot* S, const ClassLists& c, int ns, hipStream_t s) {
+  const int* n_pair = c.count + kListPair;
   const int* n_tile = c.count + kListTile;
-  const EnsWork* sep = c.work + c.off[kListSep];
-  const EnsWork* gen = c.work + c.off[kListGen];
+  const EnsWork* pairs = c.work + c.off[kListPair];
   const EnsWork* tiles = c.work + c.off[kListTile];
-  const unsigned g_sep = c.cap[kListSep], g_gen = c.cap[kListGen], g_tile = c.cap[kListTile];
-  hipLaunchKernelGGL((k_p1_ens<T, L>), dim3(g_tile), dim3(kNT), 0, s, S, n_tile, tiles);
-  for (int i = 0; i < ns; ++i) {
-    if (g_sep) hipLaunchKernelGGL((k_p2q_ens<T, L, true>), dim3(g_sep), dim3(kQNT), 0, s, S, n_sep, sep);
-    if (g_gen) hipLaunchKernelGGL((k_p2q_ens<T, L, false>), dim3(g_gen), dim3(kQNT), 0, s, S, n_gen, gen);
-    if (i + 1 < ns)
-      hipLaunchKernelGGL((k_p51_ens<T, L>), dim3(g_tile), dim3(kNT), 0, s, S, n_tile, tiles, i);
-    else
-      hipLaunchKernelGGL((k_p5_ens<T, L>), dim3(g_tile), dim3(kNT), 0, s, S, n_tile, tiles, i);
+  const unsigned g_pair = c.cap[kListPair], g_tile = c.cap[kListTile];
+  switch (lines) {
+    case 1 + CENT_P: capture_lines<T, L, CENT_P>(S, c, ns, s); break;
+    case 1 + CENT_I: capture_lines<T, L, CENT_I>(S, c, ns, s); break;
+    case 1 + CENT_C: capture_lines<T, L, CENT_C>(S, c, ns, s); break;
+    case 1 + CENT_A: capture_lines<T, L, CENT_A>(S, c, ns, s); break;
+    case 1 + CENT_F: capture_lines<T, L, CENT_F>(S, c, ns, s); break;
+    default:
+      hipLaunchKernelGGL((k_p1_ens<T, L>), dim3(g_tile), dim3(kNT), 0, s, S, n_tile, tiles);
+      for (int i = 0; i < ns; ++i) {
+        hipLaunchKernelGGL((k_p2q_ens<T, L>), dim3(g_pair), dim3(kQNT), 0, s, S, n_pair, pairs);
+        if (i + 1 < ns)
+          hipLaunchKernelGGL((k_p51_ens<T, L>), dim3(g_tile), dim3(kNT), 0, s, S, n_tile, tiles, i);
+        else
+          hipLaunchKernelGGL((k_p5_ens<T, L>), dim3(g_tile), dim3(kNT), 0, s, S, n_tile, tiles, i);
+      }
   }
   hip_check(hipGetLastError(), "ensemble sweep launch");
 }
 
 template <typename T>
-void capture_class_len(int L, const EnsSlot* S, const ClassLists& c, int ns, hipStream_t s) {
+void capture_class_len(int L, int lines, const EnsSlot* S, const ClassLists& c, int ns, hipStream_t s) {
   switch (L) {
-    case 8: capture_class<T, 8>(S, c, ns, s); break;
-    case 12: capture_class<T, 12>(S, c, ns, s); break;
-    case 16: capture_class<T, 16>(S, c, ns, s); break;
-    case 24: capture_class<T, 24>(S, c, ns, s); break;
-    case 32: capture_class<T, 32>(S, c, ns, s); break;
+    case 8: capture_class<T, 8>(lines, S, c, ns, s); break;
+    case 12: capture_class<T, 12>(lines, S, c, ns, s); break;
+    case 16: capture_class<T, 16>(lines, S, c, ns, s); break;
+    case 24: capture_class<T, 24>(lines, S, c, ns, s); break;
+    case 32: capture_class<T, 32>(lines, S, c, ns, s); break;
     default: throw Error{CFFT_ERR_UNSUPPORTED, "no ensemble kernel for this transform length"};
   }
 }
@@ -133,10 +171,10 @@ void capture_class_len(int L, const EnsSlot* S, const ClassLists& c, int ns, hip
 namespace cfft {
 
 struct EnsClass {
-  int L = 0;
+  int L = 0, lines = 0;    // transform length; line-matrix chain: 1 + centring (0: plane pairs)
   std::vector<int> parts;  // part indices
-  long off[kListsPerClass] = {0, 0, 0};      // first entry of each list in the work table
-  unsigned cap[kListsPerClass] = {0, 0, 0};  // entries each list can hold (its launches' grid)
+  long off[kListsPerClass] = {0, 0};      // first entry of each list in the work table
+  unsigned cap[kListsPerClass] = {0, 0};  // entries each list can hold (its launches' grid)
   hipStream_t st = nullptr;
   hipGraphExec_t exec = nullptr;
   hipEvent_t done = nullptr;  // end of the class's last sweep (its reads of the tables)
@@ -184,7 +222,7 @@ EnsSweep* ens_sweep_create(const std::vector<EnsPart>& parts, int ns) {
     const EnsPlanInfo i = ens_plan_info(parts[k].plan);
     require(i.path == CFFT_PATH_QS, CFFT_ERR_UNSUPPORTED, "an ensemble runs plans on path QS");
     require(!i.arith32 && !i.lanes && !i.axis_split, CFFT_ERR_UNSUPPORTED,
-            "an ensemble runs the plane-pair kernels with FP64 twiddles and the default lane split");
+            "an ensemble runs plans with FP64 twiddles, the default lane split and no per-axis chain option");
     require(i.cubic && ens_len_ok(i.L), CFFT_ERR_UNSUPPORTED,
             "an ensemble needs cubic channel grids of length 8, 12, 16, 24 or 32");
     require(i.device == e->device, CFFT_ERR_INVALID, "the plans of an ensemble share the current device");
@@ -195,24 +233,29 @@ EnsSweep* ens_sweep_create(const std::vector<EnsPart>& parts, int ns) {
     require(i.prec == e->prec, CFFT_ERR_INVALID, "the plans of an ensemble share one precision");
     e->info.push_back(i);
   }
-  // classes by transform length, larger first
-  std::vector<int> lens;
-  for (const EnsPlanInfo& i : e->info) lens.push_back(i.L);
-  std::sort(lens.begin(), lens.end(), [](int a, int b) { return a > b; });
-  lens.erase(std::unique(lens.begin(), lens.end()), lens.end());
-  e->cls.resize(lens.size());
+  // classes by transform length, larger first, and chain
+  std::vector<std::pair<int, int>> kinds;
+  for (const EnsPlanInfo& i : e->info) kinds.push_back({i.L, i.lines});
+  std::sort(kinds.begin(), kinds.end(), [](auto a, auto b) { return a > b; });
+  kinds.erase(std::unique(kinds.begin(), kinds.end()), kinds.end());
+  e->cls.resize(kinds.size());
   e->cls_of.assign(e->n, 0);
   long off = 0;
-  for (size_t c = 0; c < lens.size(); ++c) {
+  for (size_t c = 0; c < kinds.size(); ++c) {
     EnsClass& C = e->cls[c];
-    C.L = lens[c];
-    long cap[kListsPerClass] = {0, 0, 0};
+    C.L = kinds[c].first;
+    C.lines = kinds[c].second;
+    long cap[kListsPerClass] = {0, 0};
     for (int k = 0; k < e->n; ++k) {
-      if (e->info[k].L != C.L) continue;
+      if (e->info[k].L != C.L || e->info[k].lines != C.lines) continue;
       C.parts.push_back(k);
       e->cls_of[k] = (int)c;
-      cap[e->info[k].sep ? kListSep : kListGen] += e->info[k].pair_items;
-      cap[kListTile] += e->info[k].tile_items;
+      if (C.lines) {
+        cap[kListTile] += e->info[k].line_items;
+      } else {
+        cap[kListPair] += e->info[k].pair_items;
+        cap[kListTile] += e->info[k].tile_items;
+      }
     }
     for (int t = 0; t < kListsPerClass; ++t) {
       require(cap[t] < (1L << 30), CFFT_ERR_SIZE, "ensemble too large");
@@ -268,17 +311,26 @@ void ens_sweep_run(EnsSweep* e, const std::vector<EnsPart>& parts, const std::ve
     for (int t = 0; t < kListsPerClass; ++t) cnt[t] = 0;
     for (int k : C.parts) {
       const EnsPlanInfo& in = e->info[k];
-      const int lp = in.sep ? kListSep : kListGen;
-      const long pp = in.pair_items / in.batch, pt = in.tile_items / in.batch;
+      const long pp = in.pair_items / in.batch, pt = (C.lines ? in.line_items : in.tile_items) / in.batch;
       for (int b = 0; b < in.batch; ++b) {
         if (!active[k][b]) continue;
         run[c] = 1;
-        EnsWork* wp = e->work_h + C.off[lp] + cnt[lp];
-        for (long j = 0; j < pp; ++j) wp[j] = {k, (int)(b * pp + j)};
-        cnt[lp] += (int)pp;
         EnsWork* wt = e->work_h + C.off[kListTile] + cnt[kListTile];
-        for (long j = 0; j < pt; ++j) wt[j] = {k, (int)(b * pt + j)};
         cnt[kListTile] += (int)pt;
+        if (C.lines) {  // a plane's parts on one XCD, as in the plan's own launches
+          const unsigned nt = (unsigned)line_tiles(C.L);
+          for (long j = 0; j < pt; ++j) {
+            unsigned pl, part;
+            if (nt == 1) lines_item<1>((unsigned)j, (unsigned)C.L, pl, part);
+            else lines_item<2>((unsigned)j, (unsigned)C.L, pl, part);
+            wt[j] = {k, (int)((b * C.L + pl) * nt + part)};
+          }
+          continue;
+        }
+        for (long j = 0; j < pt; ++j) wt[j] = {k, (int)(b * pt + j)};
+        EnsWork* wp = e->work_h + C.off[kListPair] + cnt[kListPair];
+        for (long j = 0; j < pp; ++j) wp[j] = {k, (int)(b * pp + j)};
+        cnt[kListPair] += (int)pp;
       }
     }
   }
@@ -320,9 +372,9 @@ void ens_sweep_run(EnsSweep* e, const std::vector<EnsPart>& parts, const std::ve
       hip_check(hipStreamBeginCapture(e->cap, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
       try {
         if (e->prec == CFFT_FP64)
-          capture_class_len<double>(C.L, S, cl, e->ns, e->cap);
+          capture_class_len<double>(C.L, C.lines, S, cl, e->ns, e->cap);
         else
-          capture_class_len<float>(C.L, S, cl, e->ns, e->cap);
+          capture_class_len<float>(C.L, C.lines, S, cl, e->ns, e->cap);
       } catch (...) {
         (void)hipStreamEndCapture(e->cap, &g);
         if (g) (void)hipGraphDestroy(g);

@@ -1,6 +1,6 @@
-// Multi-plan contour sweeps: the stored (history) sweeps of several plans on
-// the plane-pair Q chain advanced together, one launch per chain stage and
-// contour step for all of them.  Plans may differ in grid, space group and
+// Multi-plan contour sweeps: the stored (history) sweeps of several path-QS
+// plans advanced together, one launch per chain stage and contour step for
+// all of them.  Plans may differ in grid, space group and
 // batch; they share precision and contour length.  No counterpart in the
 // reference (its only parallelism is threads over blocks,
 // src/execution.jl:20, 50).
@@ -11,6 +11,7 @@
 #include <cstdint>
 #include <vector>
 
+#include "lines.hpp"
 #include "pipeline.hpp"
 
 struct cfft_plan;
@@ -30,8 +31,8 @@ struct EnsSlot {
   int L;       // channel transform length H (cubic)
 };
 
-// Work entry of one workgroup: a slot and the item of its plan (a plane pair
-// or a tile).  A launch reads its entry count and entries from a work list
+// Work entry of one workgroup: a slot and the item of its plan (a plane pair,
+// a tile or a part of a plane of lines).  A launch reads its entry count and entries from a work list
 // the host fills per sweep: only the fields still active are listed, and
 // workgroups past the count exit at once.
 struct EnsWork {
@@ -59,10 +60,11 @@ struct EnsPart {
 // Host side of a plan needed by an ensemble (defined with the plan).
 struct EnsPlanInfo {
   int path, prec, arith32, device, L, cubic, batch;
-  int sep;                      // path QS: the separable Q multiply
+  int lines;                    // line-matrix chain: 1 + centring; 0: the plane-pair chain
   int lanes;                    // path QS: a lane split other than the default (0: none)
-  int axis_split;               // path QS: the per-axis chain (not run by ensembles)
+  int axis_split;               // CFFT_OPT_AXIS_SPLIT is set (ensembles refuse such plans)
   long pair_items, tile_items;  // plane-pair and tile work items of one launch
+  long line_items;              // work items of one launch of the line-matrix chain
   long M3;
 };
 EnsPlanInfo ens_plan_info(cfft_plan* p);
@@ -71,7 +73,7 @@ void ens_slot_params(cfft_plan* p, const EnsPart& part, EnsSlot* out);
 struct EnsSweep;
 // Checks the parts (path QS, FP64 twiddle arithmetic, one precision, cubic
 // channel grids of a supported length, all on the current device), sorts
-// them into classes by transform length, one stream per class, and
+// them into classes by transform length and chain, one stream per class, and
 // allocates the slot table and work lists.
 EnsSweep* ens_sweep_create(const std::vector<EnsPart>& parts, int ns);
 // The stream of the class that part k belongs to: work on part k's buffers

@@ -70,7 +70,12 @@ extern "C" {
                           * channel array); needs cubic H, L = (2,2,2), the 8
                           * representative ops diagonal with distinct sign
                           * patterns and an orthogonal cell; diffusion, steps
-                          * and the forward transform (no F_spec backward)     */
+                          * and the forward transform (no F_spec backward).
+                          * Where the multiply of a channel factors per axis
+                          * (mirror groups, half-cell glides) and H = 8, 12,
+                          * 16, 24, 32, 48 or 64, diffusion and steps run as
+                          * one real H x H matrix per channel and axis on the
+                          * FP64 matrix units, one kernel per step             */
 
 #define CFFT_FP64 0  /* all arithmetic FP64                                   */
 #define CFFT_MIXED 1 /* FP32 data/FFT/propagator, FP64 tables and reductions  */
@@ -270,35 +275,37 @@ int cfft_sweep_hist_dev(cfft_plan* plan, void* hist, const void* const* E1, cons
  * factors, step range) and replay it on the caller's stream; at most 16
  * graphs are cached per plan.  Not used while profiling is enabled. */
 #define CFFT_OPT_GRAPH 3
-/* y rows per tile of the fold / unfold kernels (P1, P5, P51): 0 (default) =
+/* y rows per tile of the fold / unfold kernels (P1, P5, P51; the line-matrix
+ * kernels of path QS have no such tiles): 0 (default) =
  * the largest power of two <= 8 dividing H1; otherwise 1, 2, 4 or 8 dividing
  * H1 (CFFT_ERR_INVALID else).  Results do not depend on it; see
  * cfft_hip.tune for timing the choices on a workload. */
 #define CFFT_OPT_TILE_ROWS 4
-/* Mixed precision on path QS: 0 (default) forms the transforms' twiddle
- * products and the fold/unfold factors in FP64 (data and butterflies FP32),
- * 1 in FP32 (about 4 % faster per step; the roundings of those factors then
- * repeat on every contour step and bias F by about 1e-6).  The plane-pair Q
- * multiply and the interaction factors are FP64 either way. */
+/* Mixed precision on path QS, plane-pair chain: 0 (default) forms the
+ * transforms' twiddle products and the fold/unfold factors in FP64 (data and
+ * butterflies FP32), 1 in FP32 (about 4 % faster per step; the roundings of
+ * those factors then repeat on every contour step and bias F by about 1e-6).
+ * The plane-pair Q multiply and the interaction factors are FP64 either way;
+ * the line-matrix kernels compute in FP64 and ignore the option. */
 #define CFFT_OPT_FP32_TWIDDLES 5
 /* Radix schedule of the path-QS plane-pair and tile transforms: the lane
  * split R1 x R2 of a length-H transform (in-lane R2-point passes, then one
  * cross-lane radix-R1 pass).  0 (default): R1 = 4 for H divisible by 16,
- * else 2; 2 selects R1 = 2 for H = 16 or 32 (results differ from the default
- * by rounding only).  Other values: CFFT_ERR_UNSUPPORTED. */
+ * else 2; 2 selects R1 = 2 for H = 16 or 32, and with it the plane-pair
+ * kernels for every plan (results differ from the default by rounding only).
+ * Other values: CFFT_ERR_UNSUPPORTED. */
 #define CFFT_OPT_FFT_LANES 6
 /* Threads per plane-pair workgroup on path QS: 0 or 256 (default), or 512
- * for H = 16, 24, 32 (same results bit for bit). */
+ * for H = 16, 24, 32 (same results bit for bit; no effect on the line-matrix
+ * kernels). */
 #define CFFT_OPT_PAIR_THREADS 7
-/* Path QS, 0 (default) or 1: the per-axis chain.  With the separable multiply
- * (orthogonal cell, translations separable in the sign pattern) the Q multiply
- * factors into one 2 x 2 mixing per axis; 1 applies the x mixing with the x
- * transforms in the unfold/fold tile kernel and the y and z mixings in a
- * kernel over single x-planes (twice the work items of the plane pairs),
- * with 32-point lines over eight lanes (other lengths: the default lane
- * split).  H = 8, 12, 16, 24 or 32, FP64 twiddle products, default lane
- * split; results differ from the default chain by rounding only.  Ensembles
- * refuse such plans.  Otherwise CFFT_ERR_UNSUPPORTED. */
+/* Path QS, 0 (default) or 1: the per-axis chain (one operator per axis
+ * instead of plane pairs).  The line-matrix kernels are that chain and every
+ * plan this option accepts runs them by default, so it changes nothing there;
+ * it is accepted for a separable multiply (orthogonal cell, translations
+ * separable in the sign pattern), H = 8, 12, 16, 24 or 32, FP64 twiddle
+ * products and the default lane split, and ensembles refuse a plan that has
+ * it set.  Otherwise CFFT_ERR_UNSUPPORTED. */
 #define CFFT_OPT_AXIS_SPLIT 8
 /* No counterpart in the reference. */
 int cfft_plan_set_option(cfft_plan* plan, int32_t key, int64_t value);
