@@ -22,7 +22,12 @@ FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 
-SOURCES = [os.path.join(CSRC, f) for f in ("cfft_hip.hip", "lines.hip", "blocks.hip", "scft.hip", "mlp.hip", "dense.hip",
+# (source, extra flags): lines.hip is compiled once per precision; its kernels
+# take their leading arguments preloaded into scalar registers
+_LINES = ["-mllvm", "-amdgpu-kernarg-preload-count=14"]
+SOURCES = [(os.path.join(CSRC, "lines.hip"), ["-DLINES_PREC=64", *_LINES]),
+           (os.path.join(CSRC, "lines.hip"), ["-DLINES_PREC=32", *_LINES])]
+SOURCES += [(os.path.join(CSRC, f), []) for f in ("cfft_hip.hip", "blocks.hip", "scft.hip", "mlp.hip", "dense.hip",
                                             "ensemble.hip", "p3c.hip", "plan.cpp")]
 
 
@@ -38,10 +43,10 @@ def build(verbose: bool = True) -> str:
     os.makedirs(objdir, exist_ok=True)
     objs, procs = [], []
     cflags = [f for f in FLAGS if f != "-shared"]
-    for src in SOURCES:
-        obj = os.path.join(objdir, os.path.basename(src) + ".o")
+    for k, (src, extra) in enumerate(SOURCES):
+        obj = os.path.join(objdir, f"{k}_{os.path.basename(src)}.o")
         objs.append(obj)
-        procs.append((src, _run([HIPCC, *cflags, "-c", "-o", obj, src], verbose)))
+        procs.append((src, _run([HIPCC, *cflags, *extra, "-c", "-o", obj, src], verbose)))
     failed = False
     for src, pr in procs:
         out, _ = pr.communicate()

@@ -48,7 +48,7 @@ struct cfft_plan {
   int qs_items = 0;  // plane-pair items per batch entry (path QS)
   int qs_sep = 0;    // path QS: translations separable in the sign pattern
   int lines_ok = 0;  // path QS: the line-matrix chain applies (a channel's multiply factors per axis)
-  int axv[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // its matrix variants (PipeP::axv)
+  unsigned long long axv = 0;  // its matrix variants (LineP::axv)
   size_t esz = 8;  // element size of the plan's real type
   hipStream_t stream = nullptr;
   // device tables
@@ -176,6 +176,7 @@ void build_lines(cfft_plan* p, const int (&tsel)[8][3]) {
       if (df != 0 && 2 * df != p->N[d]) return;
       tau[s][d] = df ? 1 : 0;
     }
+  unsigned long long axv = 0;
   for (int c = 0; c < p->n_ch; ++c) {
     auto sigma = [&](int s) {
       int v = 0;
@@ -188,14 +189,14 @@ void build_lines(cfft_plan* p, const int (&tsel)[8][3]) {
         if ((s >> d) & 1) v ^= sigma(1 << d);
       if (sigma(s) != v) return;
     }
-    p->axv[c] = 0;
-    for (int d = 0; d < 3; ++d) p->axv[c] |= (p->offs[c][d] | (sigma(1 << d) << 1)) << (2 * d);
+    for (int d = 0; d < 3; ++d)
+      axv |= (unsigned long long)(p->offs[c][d] | (sigma(1 << d) << 1)) << (6 * c + 2 * d);
   }
   // Sums in extended precision; the entries of a row are rounded to double
   // largest first, each taking the rounding error of those before it, so a
   // row keeps its sum (the gain of the k = 0 mode, which acts on every step
   // alike) to the last bit of its smallest entries.
-  const int H = p->H[0], M = 2 * H, KS = H / 4, VAR = line_variant_len(H);
+  const int H = p->H[0], M = 2 * H, VAR = line_variant_len(H);
   const long double tp = 2.0L * 3.14159265358979323846264338327950288L;
   std::vector<double> tab((size_t)12 * VAR, 0.0);
   std::vector<long double> cr(M), ci(M), T(2 * H), W(2 * H), f0(M), f1r(M), f1i(M), row(H);
@@ -241,9 +242,7 @@ void build_lines(cfft_plan* p, const int (&tsel)[8][3]) {
           for (int x : by) {
             const double e = (double)(row[x] + err);
             err += row[x] - e;
-            // lane and k-step of column x in the two contraction orders (lines.hpp)
-            const int i = d == 0 ? x % KS : x / 4, g = d == 0 ? x / KS : x % 4;
-            v[line_entry(H, r / 16, i, 16 * g + r % 16)] = e;
+            v[line_entry(H, r / 16, x / 4, 16 * (x % 4) + r % 16)] = e;
           }
         }
       }
@@ -255,6 +254,7 @@ void build_lines(cfft_plan* p, const int (&tsel)[8][3]) {
     std::lock_guard<std::recursive_mutex> guard(setup_mutex());
     hip_check(hipMemcpy(p->d_lines.p, tab.data(), p->d_lines.bytes, hipMemcpyHostToDevice), "upload line matrices");
   }
+  p->axv = axv;
   p->lines_ok = 1;
 }
 
@@ -748,7 +748,6 @@ PipeP pipe_params(cfft_plan* p, const ESel& es) {
   pp.n_rep = p->n_rep;
   pp.qs_items = p->qs_items;
   pp.qs_sep = p->qs_sep;
-  for (int c = 0; c < 8; ++c) pp.axv[c] = p->axv[c];
   return pp;
 }
 
@@ -767,7 +766,6 @@ PipeBufs pipe_bufs(cfft_plan* p, const void* f0_in, void* f0_out, void* F, bool 
   B.grep = p->d_grep.p;
   B.qmap = static_cast<const uint32_t*>(p->d_qmap.p);
   B.qsep = p->d_qsep.p;
-  B.lines = static_cast<const double*>(p->d_lines.p);
   return B;
 }
 
@@ -1006,20 +1004,45 @@ void launch_p51(cfft_plan* p, const PipeP& pp, const PipeBufs& B, int step, hipS
 // fold, z-lines into half 0 of the channels), a kernel between two steps, and
 // the last (unfold, E into f0_out).  Kernel n of a chain reads half n of the
 // channels (mod 2) and takes y-lines for even n, z-lines for odd n.
+LineP line_params(const cfft_plan* p, const PipeP& pp, const PipeBufs& B, int step, int flags) {
+  LineP l{};
+  l.ch = B.ch;
+  l.mats = static_cast<const double*>(p->d_lines.p);
+  l.axv = p->axv;
+  l.batch = p->batch;
+  l.step = step;
+  l.flags = flags | (pp.E_contig ? kLineContig : 0);
+  l.E = pp.E_contig ? static_cast<const double*>(pp.E1[0]) : nullptr;
+  l.f0_in = B.f0_in;
+  l.f0_out = B.f0_out;
+  return l;
+}
+
+LineEnt line_ents(const cfft_plan* p, const PipeP& pp) {
+  LineEnt e{};
+  for (int b = 0; b < p->batch && b < kMaxEPtr && !pp.E_contig; ++b)
+    e.ent[b] = {static_cast<const double*>(pp.E1[b]), static_cast<const double*>(pp.E2[b]), pp.sw[b]};
+  return e;
+}
+
+// kernel n of a chain
+int line_flags(int n) { return (n & 1) ? kLineFlip | kLineZ : 0; }
+
 void launch_lines_first(cfft_plan* p, const PipeP& pp, const PipeBufs& B, int step, hipStream_t s) {
   StageTimer st(p, s, CFFT_STAGE_FOLD);
-  launch_lines(p->prec, p->H[0], p->cent, kLinesOut, pp, B, step, 2, 1, s);
+  launch_lines(p->prec, p->H[0], p->cent, kLinesOut, line_params(p, pp, B, step, kLineFlip | kLineZ), line_ents(p, pp),
+               s);
 }
 
 void launch_lines_mid(cfft_plan* p, const PipeP& pp, const PipeBufs& B, int step, int n, hipStream_t s) {
   StageTimer st(p, s, CFFT_STAGE_UNFOLD_FOLD);
   const int mode = kLinesIn | kLinesOut | (B.f0_out ? kLinesStore : 0);
-  launch_lines(p->prec, p->H[0], p->cent, mode, pp, B, step, 1 + (n & 1), n & 1, s);
+  launch_lines(p->prec, p->H[0], p->cent, mode, line_params(p, pp, B, step, line_flags(n)), line_ents(p, pp), s);
 }
 
 void launch_lines_last(cfft_plan* p, const PipeP& pp, const PipeBufs& B, int step, int n, hipStream_t s) {
   StageTimer st(p, s, CFFT_STAGE_UNFOLD);
-  launch_lines(p->prec, p->H[0], p->cent, kLinesIn, pp, B, step, 1 + (n & 1), n & 1, s);
+  launch_lines(p->prec, p->H[0], p->cent, kLinesIn, line_params(p, pp, B, step, line_flags(n)), line_ents(p, pp), s);
 }
 
 // Work buffers of one diffusion call: channel spectra, the Q-multiplied
@@ -1475,7 +1498,7 @@ EnsPlanInfo ens_plan_info(cfft_plan* p) {
   i.axis_split = p->axis_split;
   i.pair_items = (long)p->qs_items * p->batch;
   i.tile_items = n_tiles(p, pipe_params(p, ESel{}));
-  i.line_items = (long)p->batch * p->H[0] * line_tiles(p->H[0]);
+  i.line_items = (long)p->batch * p->H[0] * line_parts(p->H[0]);
   i.M3 = p->M3;
   return i;
 }
@@ -1494,6 +1517,10 @@ void ens_slot_params(cfft_plan* p, const EnsPart& part, EnsSlot* out) {
   std::memset(static_cast<void*>(out), 0, sizeof(EnsSlot));
   out->p = pipe_params(p, es);
   out->B = pipe_bufs(p, nullptr, nullptr, p->d_F.p, false);
+  if (use_lines(p)) {
+    out->l = line_params(p, out->p, out->B, 0, 0);
+    out->le = line_ents(p, out->p);
+  }
   out->q = part.hist;
   out->stride = p->M3 * p->batch;
   out->L = p->H[0];

@@ -33,21 +33,24 @@ __device__ __forceinline__ const EnsSlot& ens_slot(const EnsSlot* S, int k) {
 
 // A kernel of the line-matrix chain over the listed parts (item: (plane of
 // all batch entries) * parts + part), as launched by the plan's own sweep:
-// step -1 folds slice 0, otherwise q(step + 1) goes to its slice.
+// kLinesOut alone folds slice 0, otherwise q(step + 1) goes to its slice.
 template <typename T, int L, int CENT, int MODE>
-__global__ void __launch_bounds__(64 * LineCent<CENT>::NCH) k_lines_ens(const EnsSlot* __restrict__ S, const int* __restrict__ count,
-                                                        const EnsWork* __restrict__ work, int step, int line,
-                                                        int flip) {
-  constexpr int NT = line_tiles(L);
-  __shared__ double lds[LineCent<CENT>::NCH * L * 16];
+__global__ void __launch_bounds__(64 * LineCent<CENT>::NCH, line_waves(L))
+    k_lines_ens(const EnsSlot* __restrict__ S, const int* __restrict__ count, const EnsWork* __restrict__ work,
+                int step, int flags) {
+  constexpr int NPART = line_parts(L);
+  __shared__ __align__(16) unsigned char lds[LineLds<T, L, CENT, MODE>::BYTES];
   if ((int)blockIdx.x >= *count) return;
   const EnsWork wk = work[blockIdx.x];
   const EnsSlot& s = ens_slot(S, wk.slot);
-  PipeBufs B = s.B;
-  B.f0_in = s.q;
-  if (MODE != kLinesOut) B.f0_out = static_cast<T*>(s.q) + (long)(step + 1) * s.stride;
-  const int pl = wk.item / NT;
-  ph_lines<T, L, CENT, MODE>(s.p, B, pl / L, pl % L, wk.item % NT, step, line, flip, lds);
+  const int pl = wk.item / NPART, b = pl / L;
+  LineP p = s.l;
+  p.step = step;
+  p.flags = flags;
+  p.f0_in = s.q;
+  p.f0_out = MODE == kLinesOut ? nullptr : static_cast<T*>(s.q) + (long)(step + 1) * s.stride;
+  const LineEnt::Entry e = s.le.ent[b];
+  ph_lines<T, L, CENT, MODE>(p, line_E(e, step), line_E(e, step + 1), b, pl % L, wk.item % NPART, lds);
 }
 
 // Plane pairs (FFT y, z, Q multiply, IFFT z, y) of the listed plans.
@@ -121,11 +124,11 @@ void capture_lines(const EnsSlot* S, const ClassLists& c, int ns, hipStream_t s)
   const EnsWork* w = c.work + c.off[kListTile];
   const dim3 grid(c.cap[kListTile]), block(64 * LineCent<CENT>::NCH);
   constexpr int kMid = kLinesIn | kLinesOut | kLinesStore;
-  hipLaunchKernelGGL((k_lines_ens<T, L, CENT, kLinesOut>), grid, block, 0, s, S, n, w, 0, 2, 1);
+  auto flags = [](int i) { return (i & 1) ? kLineFlip | kLineZ : 0; };
+  hipLaunchKernelGGL((k_lines_ens<T, L, CENT, kLinesOut>), grid, block, 0, s, S, n, w, 0, kLineFlip | kLineZ);
   for (int i = 0; i + 1 < ns; ++i)
-    hipLaunchKernelGGL((k_lines_ens<T, L, CENT, kMid>), grid, block, 0, s, S, n, w, i, 1 + (i & 1), i & 1);
-  const int i = ns - 1;
-  hipLaunchKernelGGL((k_lines_ens<T, L, CENT, kLinesIn>), grid, block, 0, s, S, n, w, i, 1 + (i & 1), i & 1);
+    hipLaunchKernelGGL((k_lines_ens<T, L, CENT, kMid>), grid, block, 0, s, S, n, w, i, flags(i));
+  hipLaunchKernelGGL((k_lines_ens<T, L, CENT, kLinesIn>), grid, block, 0, s, S, n, w, ns - 1, flags(ns - 1));
 }
 
 template <typename T, int L>
@@ -318,11 +321,10 @@ void ens_sweep_run(EnsSweep* e, const std::vector<EnsPart>& parts, const std::ve
         EnsWork* wt = e->work_h + C.off[kListTile] + cnt[kListTile];
         cnt[kListTile] += (int)pt;
         if (C.lines) {  // a plane's parts on one XCD, as in the plan's own launches
-          const unsigned nt = (unsigned)line_tiles(C.L);
+          const unsigned nt = (unsigned)line_parts(C.L);
           for (long j = 0; j < pt; ++j) {
             unsigned pl, part;
-            if (nt == 1) lines_item<1>((unsigned)j, (unsigned)C.L, pl, part);
-            else lines_item<2>((unsigned)j, (unsigned)C.L, pl, part);
+            lines_item(nt, (unsigned)j, (unsigned)C.L, pl, part);
             wt[j] = {k, (int)((b * C.L + pl) * nt + part)};
           }
           continue;

@@ -26,6 +26,8 @@ constexpr int kEnsMax = 64;  // plans per ensemble
 struct EnsSlot {
   PipeP p;
   PipeBufs B;  // f0_in / f0_out are set per launch from q, stride and the step
+  LineP l;     // the same for a plan on the line-matrix chain (step, flags and fields set per launch)
+  LineEnt le;
   void* q;
   long stride;
   int L;       // channel transform length H (cubic)

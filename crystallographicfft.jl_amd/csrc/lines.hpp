@@ -19,9 +19,8 @@
 // (planes of fixed z) and z-lines (planes of fixed y); each applies A_x and
 // its line matrix to its input, then unfold, E, fold at its points, then its
 // line matrix again, which leaves A_x and the other line matrix to the next
-// kernel.  A workgroup takes the line axis in full and 16 x-values of one
-// plane; A_x reads the plane's other x-values (shared by the plane's
-// workgroups through the L2).  Source and destination channels alternate
+// kernel.  A workgroup takes the line axis in full and kCW x-values of one
+// plane; A_x reads the plane's other x-values too.  Source and destination channels alternate
 // between the two halves of the plan's channel buffer.
 #pragma once
 
@@ -41,20 +40,40 @@ inline bool line_len_ok(int H) {
   return false;
 }
 
-// Matrix table (B.lines): entry [axis][variant][tile t][k-step i][lane] with
-// variant = o | (chi < 0) << 1, tiles of 16 matrix rows, H/4 k-steps.  Lane l
-// of axis 0 holds A[16 t + l % 16][(H/4) (l / 16) + i] (the contraction order
-// of rows read from memory, (H/4) consecutive values per lane), lane l of
-// axes 1, 2 holds A[16 t + l % 16][4 i + l / 16] (the order in which the
-// matrix instruction leaves its result); rows past H are 0.  An even number
-// of k-steps is stored in pairs, one 16-byte load each.
+// Interaction factors of batch entry b: e1 for steps < sw, then e2.
+struct LineEnt {
+  struct Entry {
+    const double *e1, *e2;
+    long sw;
+  } ent[kMaxEPtr];
+};
+
+// Arguments of the chain's kernels besides LineEnt, in the order the kernels
+// take them: the first 14 dwords reach a wave in scalar registers, so its
+// first loads wait for no argument fetch.
+struct LineP {
+  void* ch;                // channels: two halves of batch x n_ch x H^3 reals
+  const double* mats;      // matrix table
+  unsigned long long axv;  // matrix variant of channel c on axis d: bits 6 c + 2 d
+  int batch, step;
+  int flags;               // kLineFlip, kLineContig, kLineZ
+  const double* E;         // kLineContig: one array of batch x M^3 factors (nullptr: none)
+  const void* f0_in;
+  void* f0_out;
+};
+enum { kLineFlip = 1, kLineContig = 2, kLineZ = 4 };  // half of ch read; factors in E, not LineEnt; z-lines
+
+// Matrix table: entry [axis][variant][tile t][k-step i][lane] with variant =
+// o | (chi < 0) << 1, tiles of 16 matrix rows, H/4 k-steps; lane l holds
+// A[16 t + l % 16][4 i + l / 16], the order in which the matrix instruction
+// takes its operands and leaves its result.  Rows past H are 0.  An even
+// number of k-steps is stored in pairs, one 16-byte load each.
 constexpr int line_tiles(int H) { return (H + 15) / 16; }
 constexpr int line_variant_len(int H) { return line_tiles(H) * (H / 4) * 64; }
 constexpr int line_entry(int H, int t, int i, int lane) {
   const int KS = H / 4;
   return KS % 2 == 0 ? (t * KS + (i & ~1)) * 64 + 2 * lane + (i & 1) : (t * KS + i) * 64 + lane;
 }
-
 // The k-steps of one matrix tile for this lane.
 template <int KS>
 __device__ __forceinline__ void load_matrix(const double* __restrict__ m, int lane, double (&v)[KS]) {
@@ -70,6 +89,58 @@ __device__ __forceinline__ void load_matrix(const double* __restrict__ m, int la
 #pragma unroll
     for (int i = 0; i < KS; ++i) v[i] = m[64 * i + lane];
   }
+}
+
+// One channel of a plane, H rows of W values (all H, or half of them in each of
+// two rounds where H > 32), staged in LDS by its wave: rows are read in 16-byte
+// chunks, whole rows by neighbouring lanes (measured 63 bytes per cycle and
+// CU; the matrix operand's own pattern, 16 rows of 64 bytes per load, takes
+// 17, and loads straight into LDS issue at one per 120 cycles), and written
+// with chunk c of row r at chunk (c + s(r)) mod the row's chunks, s(r) chosen
+// so that the 16 rows an operand read touches lie on different banks.
+template <typename T, int H>
+struct LineStage {
+  static constexpr int E = 16 / (int)sizeof(T);        // values per chunk
+  static constexpr int W = H <= 32 ? H : H / 2, ROUNDS = H / W;
+  static constexpr int C = W / E;                      // chunks per row
+  static constexpr int N = H * C, NI = (N + 63) / 64;  // chunks, loads of 64 lanes
+  static constexpr int G = C % 16 == 0 ? 16 : (C % 8 == 0 ? 8 : (C % 4 == 0 ? 4 : (C % 2 == 0 ? 2 : 1)));
+  static constexpr int BYTES = 16 * N;
+  static_assert(W % E == 0 && W % 4 == 0, "rows of whole chunks and k-steps");
+  __device__ static __forceinline__ int shift(int row) { return row * G / 16; }
+};
+
+template <typename T, int H>
+struct LineRows {  // a round's chunks on their way to LDS
+  typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
+  vec v[LineStage<T, H>::NI];
+};
+template <typename T, int H>
+__device__ __forceinline__ void load_rows(const T* __restrict__ src, unsigned rs, int lane, LineRows<T, H>& q) {
+  typedef LineStage<T, H> S;
+#pragma unroll
+  for (int j = 0; j < S::NI; ++j) {
+    const int k0 = 64 * j + lane, k = S::N % 64 == 0 || k0 < S::N ? k0 : S::N - 1;
+    q.v[j] = *reinterpret_cast<const typename LineRows<T, H>::vec*>(
+        src + ((unsigned)(k / S::C) * rs + (unsigned)(k % S::C * S::E)));
+  }
+}
+template <typename T, int H>
+__device__ __forceinline__ void stage_rows(const LineRows<T, H>& q, int lane, unsigned char* lds) {
+  typedef LineStage<T, H> S;
+#pragma unroll
+  for (int j = 0; j < S::NI; ++j) {
+    const int k = 64 * j + lane, row = k / S::C, c = (k % S::C + S::shift(row)) % S::C;
+    if (S::N % 64 == 0 || k < S::N) reinterpret_cast<typename LineRows<T, H>::vec*>(lds)[row * S::C + c] = q.v[j];
+  }
+}
+
+// Value x < W of row `row`.
+template <typename T, int H>
+__device__ __forceinline__ double staged(const unsigned char* lds, int row, int x) {
+  typedef LineStage<T, H> S;
+  const int c = (x / S::E + S::shift(row)) % S::C;
+  return (double)reinterpret_cast<const T*>(lds)[(row * S::C + c) * S::E + x % S::E];
 }
 
 // Channels of a lattice centring (plan.hpp's Centering) as a group of
@@ -116,26 +187,21 @@ __host__ __device__ constexpr int line_class(int e) {
   return v;
 }
 
-// KS consecutive values at p (aligned to their power-of-two part) as doubles.
-template <typename T, int KS>
-__device__ __forceinline__ void load_run(const T* __restrict__ p, double (&v)[KS]) {
-  constexpr int BYTES = KS * (int)sizeof(T);
-  constexpr int VB = BYTES % 16 == 0 ? 16 : (BYTES % 8 == 0 ? 8 : 4);
-  constexpr int VE = VB / (int)sizeof(T);
-  typedef T vec __attribute__((ext_vector_type(VE)));
-  if constexpr (VE == 1) {
-#pragma unroll
-    for (int i = 0; i < KS; ++i) v[i] = (double)p[i];
-  } else {
-    vec t[KS / VE];
-#pragma unroll
-    for (int i = 0; i < KS / VE; ++i) t[i] = reinterpret_cast<const vec*>(p)[i];
-#pragma unroll
-    for (int i = 0; i < KS / VE; ++i)
-#pragma unroll
-      for (int j = 0; j < VE; ++j) v[i * VE + j] = (double)t[i][j];
-  }
-}
+enum { kLinesIn = 1, kLinesOut = 2, kLinesStore = 4 };
+
+// x-values per workgroup: the matrix instructions' tile.  Measured against 8
+// (every CU at work from half the fields, half of each tile wasted) and 32
+// (a plane's rows read once): Im-3m 128^3 FP64 at 1, 2, 8, 16 fields 5.58,
+// 6.01, 12.1 us (8), 5.75, 6.11, 8.9, 15.7 us (16), 7.7, 8.1, 9.6, 14.8 us (32).
+constexpr int kCW = 16;
+constexpr int line_parts(int H) { return (H + kCW - 1) / kCW; }
+
+// LDS of a workgroup: per channel its staged plane, then its H x kCW points.
+template <typename T, int H, int CENT, int MODE>
+struct LineLds {
+  static constexpr int PTS = 8 * H * kCW, ST = (MODE & kLinesIn) ? LineStage<T, H>::BYTES : 0;
+  static constexpr int CH = PTS > ST ? PTS : ST, BYTES = LineCent<CENT>::NCH * CH;
+};
 
 template <int N>
 __device__ __forceinline__ void wht(double (&v)[N]) {
@@ -150,197 +216,259 @@ __device__ __forceinline__ void wht(double (&v)[N]) {
       }
 }
 
-// One point between two steps: channel values g -> corner values (unfold,
-// factor eo), to f[off of the corner] when ST, times en, folded back into g.
-// Without IN the corner values are f_in; without OUT g is left alone.  No
-// contraction: every kernel that inlines this rounds alike.
-template <typename T, int H, int CENT, bool IN, bool OUT, bool ST>
-__device__ __forceinline__ void line_point(double (&g)[LineCent<CENT>::NCH], const double (&f_in)[8],
-                                           const double (&eo)[8], const double (&en)[8], T* __restrict__ f,
+// VX neighbouring points (x, x + 1) between two steps: channel values g ->
+// corner values (unfold, factor eo), to f at the points' offset `at` when ST,
+// times en, folded back into g.  Without IN the corner values are f_in;
+// without OUT g is left alone.  No contraction: every kernel that inlines
+// this rounds alike.
+template <typename T, int H, int CENT, int VX, bool IN, bool OUT, bool ST>
+__device__ __forceinline__ void line_point(double (&g)[LineCent<CENT>::NCH][VX], const double (&f_in)[8][VX],
+                                           const double (&eo)[8][VX], const double (&en)[8][VX], T* __restrict__ f,
                                            unsigned at) {
 #pragma clang fp contract(off)
   constexpr int NCH = LineCent<CENT>::NCH;
   constexpr unsigned M = 2 * H;
-  if constexpr (IN) {
-    wht<NCH>(g);
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) g[c] = 0.125 * g[c];
-  }
-  double h[NCH];
-#pragma unroll
-  for (int c = 0; c < NCH; ++c) h[c] = 0.0;
+  typedef T vec __attribute__((ext_vector_type(VX)));
+  double u[VX][NCH], h[VX][NCH];
   bool seen[NCH] = {};
+#pragma unroll
+  for (int v = 0; v < VX; ++v) {
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      u[v][c] = IN ? g[c][v] : 0.0;
+      h[v][c] = 0.0;
+    }
+    if constexpr (IN) {
+      wht<NCH>(u[v]);
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) u[v][c] = 0.125 * u[v][c];
+    }
+  }
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const int k = line_class<CENT>(e);
-    const double u = IN ? g[k] * eo[e] : f_in[e];
-    if constexpr (ST) {
-      T* q = f + at + (unsigned)(((e & 1) + ((e >> 1) & 1) * M + (e >> 2) * M * M) * H);
-      if constexpr (OUT) __builtin_nontemporal_store((T)u, q);  // a stored sweep's slice: read after the sweep only
-      else *q = (T)u;
+    vec out;
+#pragma unroll
+    for (int v = 0; v < VX; ++v) {
+      const double q = IN ? u[v][k] * eo[e][v] : f_in[e][v];
+      out[v] = (T)q;
+      if constexpr (OUT) {
+        const double w = q * en[e][v];
+        h[v][k] = seen[k] ? h[v][k] + w : w;
+      }
     }
-    if constexpr (OUT) {
-      const double w = u * en[e];
-      h[k] = seen[k] ? h[k] + w : w;
-      seen[k] = true;
+    seen[k] = true;
+    if constexpr (ST) {
+      vec* q = reinterpret_cast<vec*>(f + at + (unsigned)(((e & 1) + ((e >> 1) & 1) * M + (e >> 2) * M * M) * H));
+      if constexpr (OUT) __builtin_nontemporal_store(out, q);  // a stored sweep's slice: read after the sweep only
+      else *q = out;
     }
   }
   if constexpr (OUT) {
-    wht<NCH>(h);
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) g[c] = h[c];
+    for (int v = 0; v < VX; ++v) {
+      wht<NCH>(h[v]);
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) g[c][v] = h[v][c];
+    }
   }
 }
 
-// The 8 corner values of the point at offset `at` of one M^3 array.
-template <typename T, int H>
-__device__ __forceinline__ void load_corners(const T* __restrict__ f, unsigned at, double (&v)[8]) {
+// Corner e of the VX points at offset `at` of one M^3 array.
+template <typename T, int H, int VX>
+__device__ __forceinline__ void load_corner(const T* __restrict__ f, unsigned at, int e, double (&v)[VX]) {
   constexpr unsigned M = 2 * H;
+  typedef T vec __attribute__((ext_vector_type(VX)));
+  const unsigned corner = (unsigned)(((e & 1) + ((e >> 1) & 1) * M + (e >> 2) * M * M) * H);
+  const vec t = *reinterpret_cast<const vec*>(f + at + corner);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = (double)f[at + (unsigned)(((e & 1) + ((e >> 1) & 1) * M + (e >> 2) * M * M) * H)];
+  for (int i = 0; i < VX; ++i) v[i] = (double)t[i];
 }
 
-enum { kLinesIn = 1, kLinesOut = 2, kLinesStore = 4 };
+template <int VX>
+__device__ __forceinline__ void ones(double (&v)[8][VX]) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+#pragma unroll
+    for (int i = 0; i < VX; ++i) v[e][i] = 1.0;
+}
 
 // One workgroup of n_ch waves (wave c: channel c): the points (line position
-// a < H, x = 16 part + 0..15) of plane `plane` of batch entry b.  line = 1:
-// y-lines of the plane z = plane; line = 2: z-lines of the plane y = plane.
-// MODE: kLinesIn: the input is the channels at half `flip` of B.ch, A_x and
-// the line matrix applied (else the field B.f0_in); kLinesOut: folded, the
-// line matrix applied, stored to the other half; kLinesStore (and always
-// without kLinesOut): the field after E of `step` goes to B.f0_out.
+// a < H, x = kCW part + 0 .. kCW - 1) of plane `plane` of batch entry b, with
+// the entry's factors at E of `step` (Eo) and of step + 1 (En).  y-lines of
+// the plane z = plane, or (kLineZ) z-lines of the plane y = plane.  MODE:
+// kLinesIn: the input is the channels, A_x and the line matrix applied (else
+// the field f0_in); kLinesOut: folded, the line matrix applied, stored to the
+// other half; kLinesStore (and always without kLinesOut): the field after Eo
+// goes to f0_out.
 //
-// Every load is issued before the first use: per plane and step the
-// dependent chain is one memory latency, three passes of H/16 * H/4 matrix
-// instructions (64 cycles each) and two LDS exchanges.  Loads behind
-// per-value tests of the factor pointers cost 9300 of the kernel's 17000
-// cycles at H = 32; tested once per array they overlap.
+// A workgroup's time is a memory latency and three passes of H/16 * H/4
+// matrix instructions of 64 cycles, so the loads are ordered by use: rows,
+// A_x, the line matrix, and the factors between the matrix instructions of
+// the second pass.  No value test guards a load (the factor pointers are
+// tested once per array): loads behind per-value tests cost 9300 of 17000
+// cycles at H = 32.
 template <typename T, int H, int CENT, int MODE>
-__device__ __forceinline__ void ph_lines(const PipeP& p, const PipeBufs& B, int b, int plane, int part, int step,
-                                         int line, int flip, double* lds) {
+__device__ __forceinline__ void ph_lines(const LineP& p, const double* Eo, const double* En, int b, int plane,
+                                         int part, unsigned char* lds_raw) {
   constexpr int NCH = LineCent<CENT>::NCH;
   constexpr bool IN = (MODE & kLinesIn) != 0, OUT = (MODE & kLinesOut) != 0, ST = (MODE & kLinesStore) != 0 || !OUT;
   constexpr int NT = line_tiles(H), KS = H / 4, VAR = line_variant_len(H);
-  constexpr int NTH = 64 * NCH, NP = 16 * H, NPT = (NP + NTH - 1) / NTH;
+  constexpr int NTH = 64 * NCH, VX = kCW * H > NTH ? 2 : 1, XV = kCW / VX;  // VX neighbouring points per thread
+  constexpr int NP = kCW * H / VX, NPT = (NP + NTH - 1) / NTH;
+  constexpr bool FULL = H % kCW == 0;  // no columns past H
   constexpr unsigned M = 2 * H, H2 = (unsigned)H * H, H3 = H2 * H;
   constexpr long M3 = 8L * H3;
+  typedef double vecd __attribute__((ext_vector_type(VX)));
+  typedef LineStage<T, H> S;
   const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
   const int c = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int x0 = 16 * part;
+  const int x0 = kCW * part, line = (p.flags & kLineZ) ? 2 : 1, flip = p.flags & kLineFlip;
   const long half = (long)p.batch * NCH * H3;
   const long cb = ((long)b * NCH + c) * H3 + (line == 1 ? (unsigned)plane * H2 : (unsigned)plane * H);
   const unsigned rs = line == 1 ? (unsigned)H : H2;
   const unsigned sy = line == 1 ? M : M * M, sp = line == 1 ? M * M : M;  // strides of line position and plane
-  const int av = p.axv[c];
+  const int av = (int)(p.axv >> (6 * c));
 
-  double gv[NT][KS], mx[KS], ml[NT][KS];
+  // a wave's rows are staged in the bytes that then hold its channel's points
+  unsigned char* own = lds_raw + c * LineLds<T, H, CENT, MODE>::CH;
+  double* lds = reinterpret_cast<double*>(lds_raw);
+  constexpr int LC = LineLds<T, H, CENT, MODE>::CH / 8;  // doubles per channel
+  double mx[KS], ml[NT][KS];
+  const T* src = static_cast<const T*>(p.ch) + flip * half + cb;
+  LineRows<T, H> rows;
   if constexpr (IN) {
-    const T* src = static_cast<const T*>(B.ch) + flip * half + cb;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int row = 16 * t + r;
-      load_run<T, KS>(src + ((unsigned)(H % 16 == 0 || row < H ? row : H - 1) * rs + (unsigned)(KS * g)), gv[t]);
-    }
+    load_rows<T, H>(src, rs, lane, rows);
+    load_matrix<KS>(p.mats + (av & 3) * VAR + part * (KS * 64), lane, mx);
   }
-  const double* Eo = pipe_E(p, b, step, M3);
-  const double* En = IN ? pipe_E(p, b, step + 1, M3) : Eo;
   const bool other_E = IN && OUT && En != Eo;
-  double eo[NPT][8], en[NPT][8];  // en: the factor of the fold when it is another array (or the field, without IN)
+  const double* tl = p.mats + (line * 4 + ((av >> (2 * line)) & 3)) * VAR;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) load_matrix<KS>(tl + t * (KS * 64), lane, ml[t]);
+  // en: the factor of the fold when it is another array (or the field, without IN)
+  double eo[NPT][8][VX], en[NPT][8][VX];
   unsigned at[NPT];
 #pragma unroll
   for (int k = 0; k < NPT; ++k) {
     const int pt0 = (int)threadIdx.x + k * NTH, pt = NP % NTH == 0 || pt0 < NP ? pt0 : NP - 1;
-    const int xx = x0 + (pt & 15);
-    at[k] = (unsigned)(H % 16 == 0 || xx < H ? xx : H - 1) + (unsigned)(pt >> 4) * sy + (unsigned)plane * sp;
+    const int xx = x0 + VX * (pt % XV);
+    at[k] = (unsigned)(FULL || xx < H ? xx : H - VX) + (unsigned)(pt / XV) * sy + (unsigned)plane * sp;
+    ones<VX>(eo[k]);
   }
-  if (Eo) {
+  if constexpr (!IN) {
+    if (Eo) {
 #pragma unroll
-    for (int k = 0; k < NPT; ++k) load_corners<double, H>(Eo, at[k], eo[k]);
-  } else {
+      for (int k = 0; k < NPT; ++k)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) load_corner<double, H, VX>(Eo, at[k], e, eo[k][e]);
+    }
 #pragma unroll
     for (int k = 0; k < NPT; ++k)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) eo[k][e] = 1.0;
+      for (int e = 0; e < 8; ++e)
+        load_corner<T, H, VX>(static_cast<const T*>(p.f0_in) + b * M3, at[k], e, en[k][e]);
   }
-  if constexpr (IN) {
-    load_matrix<KS>(B.lines + (long)(av & 3) * VAR + part * (KS * 64), lane, mx);
-    if (other_E) {
-      if (En) {
-#pragma unroll
-        for (int k = 0; k < NPT; ++k) load_corners<double, H>(En, at[k], en[k]);
-      } else {
-#pragma unroll
-        for (int k = 0; k < NPT; ++k)
-#pragma unroll
-          for (int e = 0; e < 8; ++e) en[k][e] = 1.0;
-      }
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < NPT; ++k) load_corners<T, H>(static_cast<const T*>(B.f0_in) + b * M3, at[k], en[k]);
-  }
-  const double* tl = B.lines + ((long)line * 4 + ((av >> (2 * line)) & 3)) * VAR;
-#pragma unroll
-  for (int t = 0; t < NT; ++t) load_matrix<KS>(tl + t * (KS * 64), lane, ml[t]);
 
   if constexpr (IN) {
+    stage_rows<T, H>(rows, lane, own);
     mfma_d4 a1[NT], a2[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       a1[t] = mfma_d4{0.0, 0.0, 0.0, 0.0};
       a2[t] = mfma_d4{0.0, 0.0, 0.0, 0.0};
     }
-    // A_x: rows of the plane (line positions) times the part's 16 columns of A_x^T
+    // A_x: rows of the plane (line positions) times 16 columns of A_x^T
 #pragma unroll
-    for (int i = 0; i < KS; ++i)
+    for (int i = 0; i < KS; ++i) {
+      if (i > 0 && 4 * i % S::W == 0) {  // the next round's columns, over the ones just read
+        load_rows<T, H>(src + 4 * i, rs, lane, rows);
+        stage_rows<T, H>(rows, lane, own);
+      }
 #pragma unroll
-      for (int t = 0; t < NT; ++t) a1[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(gv[t][i], mx[i], a1[t], 0, 0, 0);
+      for (int t = 0; t < NT; ++t) {
+        const int row = 16 * t + r;
+        const double gv = staged<T, H>(own, H % 16 == 0 || row < H ? row : H - 1, 4 * i % S::W + g);
+        a1[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(gv, mx[i], a1[t], 0, 0, 0);
+      }
+    }
     // the line matrix: result register j of tile t is line position
     // 16 t + 4 j + l / 16, the B operand of k-step 4 t + j
 #pragma unroll
-    for (int i = 0; i < KS; ++i)
+    for (int i = 0; i < KS; ++i) {
+      // the factors' loads between the matrix instructions: a wave that issues
+      // them ahead of phase 1 stands still until the CU has taken them
+      __builtin_amdgcn_sched_barrier(0);
+      if (Eo) {
+#pragma unroll
+        for (int j = i * NPT * 8 / KS; j < (i + 1) * NPT * 8 / KS; ++j)
+          load_corner<double, H, VX>(Eo, at[j / 8], j % 8, eo[j / 8][j % 8]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         a2[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ml[t][i], a1[i / 4][i % 4], a2[t], 0, 0, 0);
+    }
+    if (other_E) {
+#pragma unroll
+      for (int k = 0; k < NPT; ++k) ones<VX>(en[k]);
+      if (En) {
+#pragma unroll
+        for (int k = 0; k < NPT; ++k)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) load_corner<double, H, VX>(En, at[k], e, en[k][e]);
+      }
+    }
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (16 * t + 4 * j < H) lds[(c * H + 16 * t + 4 * j + g) * 16 + r] = a2[t][j];
+        if (16 * t + 4 * j < H) lds[c * LC + (16 * t + 4 * j + g) * kCW + r] = a2[t][j];
     __syncthreads();
   }
-  T* f_out = static_cast<T*>(B.f0_out) + b * M3;
+  T* f_out = static_cast<T*>(p.f0_out) + b * M3;
+  vecd* ldv = reinterpret_cast<vecd*>(lds);
 #pragma unroll
   for (int k = 0; k < NPT; ++k) {
     const int pt = (int)threadIdx.x + k * NTH;
     if (NP % NTH != 0 && pt >= NP) continue;
-    double v[NCH];
+    double v[NCH][VX];
     if constexpr (IN) {
 #pragma unroll
-      for (int cc = 0; cc < NCH; ++cc) v[cc] = lds[cc * NP + pt];
+      for (int cc = 0; cc < NCH; ++cc) {
+        const vecd w = ldv[cc * (LC / VX) + pt];
+#pragma unroll
+        for (int i = 0; i < VX; ++i) v[cc][i] = w[i];
+      }
     }
     // columns past H (part-filled tiles) hold no field point
-    const bool out = ST && (H % 16 == 0 || x0 + (pt & 15) < H);
-    auto point = [&](const double(&a)[8], const double(&w)[8]) {
-      if (out) line_point<T, H, CENT, IN, OUT, ST>(v, en[k], a, w, f_out, at[k]);
-      else line_point<T, H, CENT, IN, OUT, false>(v, en[k], a, w, f_out, at[k]);
+    const bool out = ST && (FULL || x0 + VX * (pt % XV) < H);
+    auto point = [&](const double(&a)[8][VX], const double(&w)[8][VX]) {
+      if (out) line_point<T, H, CENT, VX, IN, OUT, ST>(v, en[k], a, w, f_out, at[k]);
+      else line_point<T, H, CENT, VX, IN, OUT, false>(v, en[k], a, w, f_out, at[k]);
     };
     if (other_E) {
       point(eo[k], en[k]);
     } else {
       // taken here, not where the loads are issued: a copy of eo into en's
       // registers up there would wait for it
-      double w[8];
+      double w[8][VX];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        w[e] = eo[k][e];
-        asm volatile("" : "+v"(w[e]));
-      }
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int i = 0; i < VX; ++i) {
+          w[e][i] = eo[k][e][i];
+          asm volatile("" : "+v"(w[e][i]));
+        }
       point(eo[k], w);
     }
     if constexpr (OUT) {
 #pragma unroll
-      for (int cc = 0; cc < NCH; ++cc) lds[cc * NP + pt] = v[cc];
+      for (int cc = 0; cc < NCH; ++cc) {
+        vecd w;
+#pragma unroll
+        for (int i = 0; i < VX; ++i) w[i] = v[cc][i];
+        ldv[cc * (LC / VX) + pt] = w;
+      }
     }
   }
   if constexpr (OUT) {
@@ -350,17 +478,18 @@ __device__ __forceinline__ void ph_lines(const PipeP& p, const PipeBufs& B, int 
     for (int t = 0; t < NT; ++t) a3[t] = mfma_d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int i = 0; i < KS; ++i) {
-      const double w = lds[(c * H + 4 * i + g) * 16 + r];
+      const double w = lds[c * LC + (4 * i + g) * kCW + r];
 #pragma unroll
       for (int t = 0; t < NT; ++t) a3[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ml[t][i], w, a3[t], 0, 0, 0);
     }
-    T* dst = static_cast<T*>(B.ch) + (1 - flip) * half + cb;
-    if (H % 16 == 0 || x0 + r < H) {
+    T* dst = static_cast<T*>(p.ch) + (1 - flip) * half + cb;
+    const int x = x0 + r;
+    if (FULL || x < H) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (16 * t + 4 * j < H) dst[(unsigned)(16 * t + 4 * j + g) * rs + (unsigned)(x0 + r)] = (T)a3[t][j];
+          if (16 * t + 4 * j < H) dst[(unsigned)(16 * t + 4 * j + g) * rs + (unsigned)x] = (T)a3[t][j];
     }
   }
 }
@@ -368,28 +497,48 @@ __device__ __forceinline__ void ph_lines(const PipeP& p, const PipeBufs& B, int 
 // Workgroup -> (plane of all batch entries, x part).  The parts of a plane
 // read the whole plane: blocks go to the 8 XCDs round robin, so the parts of
 // plane 8 j + i are the blocks of that i in group j and share an L2.
-template <int NT>
-__host__ __device__ __forceinline__ void lines_item(unsigned blk, unsigned n_planes, unsigned& pl, unsigned& part) {
-  if (NT > 1 && n_planes % 8 == 0) {
+__host__ __device__ __forceinline__ void lines_item(unsigned parts, unsigned blk, unsigned n_planes, unsigned& pl,
+                                                    unsigned& part) {
+  if (parts > 1 && n_planes % 8 == 0) {
     const unsigned j = blk >> 3;
-    part = j % NT;
-    pl = (j / NT) * 8 + (blk & 7);
+    part = j % parts;
+    pl = (j / parts) * 8 + (blk & 7);
   } else {
-    part = blk % NT;
-    pl = blk / NT;
+    part = blk % parts;
+    pl = blk / parts;
   }
 }
 
+// Factors of batch entry b at `step`.
+__device__ __forceinline__ const double* line_E(const LineEnt::Entry& e, int step) { return step < e.sw ? e.e1 : e.e2; }
+
+// Three waves per SIMD where the registers allow it: below that the compiler
+// moves the accumulators through the second register file (Im-3m 128^3, 2
+// fields FP64 6.1 -> 5.8 us, 16 fields mixed 13.6 -> 11.9).
+constexpr int line_waves(int H) { return H <= 32 ? 3 : 1; }
+
 template <typename T, int H, int CENT, int MODE>
-__global__ void __launch_bounds__(64 * LineCent<CENT>::NCH) k_lines(PipeP p, PipeBufs B, int step, int line, int flip) {
-  __shared__ double lds[LineCent<CENT>::NCH * H * 16];
+__global__ void __launch_bounds__(64 * LineCent<CENT>::NCH, line_waves(H))
+    k_lines(void* ch, const double* mats, unsigned long long axv, int batch, int step, int flags, const double* E,
+            const void* f0_in, void* f0_out, LineEnt ents) {
+  __shared__ __align__(16) unsigned char lds[LineLds<T, H, CENT, MODE>::BYTES];
+  constexpr long M3 = 8L * H * H * H;
   unsigned pl, part;
-  lines_item<line_tiles(H)>(blockIdx.x, (unsigned)(p.batch * H), pl, part);
-  ph_lines<T, H, CENT, MODE>(p, B, (int)(pl / H), (int)(pl % H), (int)part, step, line, flip, lds);
+  lines_item(line_parts(H), blockIdx.x, (unsigned)(batch * H), pl, part);
+  const int b = (int)(pl / H);
+  const LineEnt::Entry ent = ents.ent[(flags & kLineContig) ? 0 : b];
+  const double* all = E ? E + b * M3 : nullptr;
+  const double* Eo = (flags & kLineContig) ? all : line_E(ent, step);
+  const double* En = (flags & kLineContig) ? all : line_E(ent, step + 1);
+  ph_lines<T, H, CENT, MODE>(LineP{ch, mats, axv, batch, step, flags, E, f0_in, f0_out}, Eo, En, b, (int)(pl % H),
+                                 (int)part, lds);
 }
 
 // Launches k_lines over every plane of the plan (lines.hip).
-void launch_lines(int prec, int H, int cent, int mode, const PipeP& p, const PipeBufs& B, int step, int line,
-                  int flip, hipStream_t s);
+template <typename T>
+void launch_lines_prec(int H, int cent, int mode, const LineP& p, const LineEnt& e, hipStream_t s);
+extern template void launch_lines_prec<double>(int, int, int, const LineP&, const LineEnt&, hipStream_t);
+extern template void launch_lines_prec<float>(int, int, int, const LineP&, const LineEnt&, hipStream_t);
+void launch_lines(int prec, int H, int cent, int mode, const LineP& p, const LineEnt& e, hipStream_t s);
 
 }  // namespace cfft

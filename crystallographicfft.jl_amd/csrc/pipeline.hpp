@@ -42,7 +42,6 @@ struct PipeP {
   long n_rep;           // orbit representatives (path QR)
   int qs_items;         // plane-pair work items per batch entry (path QS)
   int qs_sep;           // path QS: t_{s,d} depends on bit d of s only
-  int axv[8];           // line-matrix chain: matrix variant of channel c on axis d, bits 2d, 2d + 1
 };
 
 struct PipeBufs {
@@ -58,7 +57,6 @@ struct PipeBufs {
   const void* grep;      // path QR: Q-multiplied values at the orbit representatives
   const uint32_t* qmap;  // path QR: element -> rep (bits 0-19) | phase exponent << 20
   const void* qsep;      // path QS: axis factors F[d][s][q] (cx<double>, 3 x 8 x M0)
-  const double* lines;   // path QS: matrices of the line-matrix chain (lines.hpp)
 };
 
 template <int LEN, int NT = kNT, int LANES = 0>
