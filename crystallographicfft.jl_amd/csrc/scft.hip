@@ -66,26 +66,64 @@ __global__ void k_expw(const double* __restrict__ w, double* __restrict__ E, dou
 // holds nf fields; the instance's q(j) is field qf, its q+(j) field qf + 1):
 //   uA = sum_{j<=nA} wa_j q(j) q+(ns-j),  uB = sum_{j>=nA} wb_{j-nA} q(j) q+(ns-j);
 // partial sums of q(ns) and q+(ns) for Q.
+// A workgroup takes 64 points at a time, each of its four waves a quarter of
+// the contour, with kDJ contour points' loads in flight; the quarters are
+// added through LDS.  One thread per point left a 64^3 melt (32 K points) at
+// 128 workgroups of one serial chain of 101 loads: 55 us.
+constexpr int kDJ = 8;
 template <typename T>
 __global__ void __launch_bounds__(kRB) k_density(const T* __restrict__ hist, long M3, int nf, int qf, int ns,
                                                  int nA, const double* __restrict__ wa,
                                                  const double* __restrict__ wb, double* __restrict__ u,
                                                  double* __restrict__ part) {
+  constexpr int NW = kRB / 64;
+  __shared__ double ab[NW][2][64];
   double acc[2] = {0.0, 0.0};
   const T* hq = hist + (long)qf * M3;
   const T* hp = hist + (long)(qf + 1) * M3;
   const long sl = (long)nf * M3;
-  for (long x = blockIdx.x * (long)kRB + threadIdx.x; x < M3; x += (long)gridDim.x * kRB) {
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int j0 = (int)((long)w * (ns + 1) / NW), j1 = (int)((long)(w + 1) * (ns + 1) / NW);
+  for (long c = blockIdx.x; c * 64 < M3; c += gridDim.x) {
+    const long x0 = c * 64 + lane;
+    const bool ok = x0 < M3;
+    const long x = ok ? x0 : M3 - 1;
     double a = 0.0, b = 0.0;
-    for (int j = 0; j <= ns; ++j) {
-      const double pr = (double)hq[j * sl + x] * (double)hp[(ns - j) * sl + x];
-      if (j <= nA) a += wa[j] * pr;
-      if (j >= nA) b += wb[j - nA] * pr;
+    for (int js = j0; js < j1; js += kDJ) {
+      double q[kDJ], p[kDJ], va[kDJ], vb[kDJ];
+#pragma unroll
+      for (int k = 0; k < kDJ; ++k) {
+        const int j = js + k < j1 ? js + k : j1 - 1;  // unconditional loads
+        q[k] = (double)hq[j * sl + x];
+        p[k] = (double)hp[(ns - j) * sl + x];
+        va[k] = wa[j <= nA ? j : nA];
+        vb[k] = wb[j >= nA ? j - nA : 0];
+      }
+#pragma unroll
+      for (int k = 0; k < kDJ; ++k) {
+        const int j = js + k;
+        if (j >= j1) break;
+        const double pr = q[k] * p[k];
+        if (j <= nA) a += va[k] * pr;
+        if (j >= nA) b += vb[k] * pr;
+      }
     }
-    u[x] = a;
-    u[M3 + x] = b;
-    acc[0] += (double)hq[ns * sl + x];
-    acc[1] += (double)hp[ns * sl + x];
+    ab[w][0][lane] = a;
+    ab[w][1][lane] = b;
+    __syncthreads();
+    if (w < 2) {  // wave 0: uA and the sum of q(ns); wave 1: uB and of q+(ns)
+      double s = ab[0][w][lane];
+#pragma unroll
+      for (int k = 1; k < NW; ++k) s += ab[k][w][lane];
+      if (ok) {
+        u[w * M3 + x] = s;
+        const double qe = (double)(w == 0 ? hq : hp)[ns * sl + x];
+        if (w == 0) acc[0] += qe;
+        else acc[1] += qe;
+      }
+    }
+    __syncthreads();
   }
   block_sum<2>(acc, part);
 }
@@ -327,10 +365,10 @@ template <typename T>
 void update_inst(cfft_scft* c, int i, hipStream_t st) {
   ScftInst& s = *c->in[i];
   const long M3 = c->M3;
-  const unsigned nb = red_blocks(M3);
+  const unsigned nb = red_blocks(M3), nd = (unsigned)std::min<long>(kMaxRed, std::max<long>(1, nblk(M3, 64)));
   double* tot = static_cast<double*>(c->tot.p) + (long)i * kTot;
   double* phi = static_cast<double*>(c->project ? c->phi_raw.p : s.phi.p);
-  hipLaunchKernelGGL(k_density<T>, dim3(nb), dim3(kRB), 0, st, static_cast<const T*>(c->hist.p), M3,
+  hipLaunchKernelGGL(k_density<T>, dim3(nd), dim3(kRB), 0, st, static_cast<const T*>(c->hist.p), M3,
                      2 * (int)c->in.size(), 2 * i, c->ns, s.nA, static_cast<const double*>(s.wa.p),
                      static_cast<const double*>(s.wb.p), phi, static_cast<double*>(c->dpart.p));
   hip_check(hipGetLastError(), "k_density");
@@ -339,7 +377,7 @@ void update_inst(cfft_scft* c, int i, hipStream_t st) {
     if (rc != CFFT_OK) throw Error{rc, g_last_error};
   }
   hipLaunchKernelGGL(k_total<2>, dim3(2), dim3(kRB), 0, st, static_cast<const double*>(c->dpart.p),
-                     (int)nb, tot);
+                     (int)nd, tot);
   hip_check(hipGetLastError(), "k_total");
   // the newest history slot and the Gram row over the ring
   const int slot = s.next_slot;
