@@ -212,6 +212,32 @@ struct TilePts {
   static constexpr int NPT = (L0 * 8 + kNT - 1) / kNT;
 };
 
+// A product rounded on its own, never fused into the sum it feeds: the fold,
+// the unfold and the two fused then round alike.
+__device__ __forceinline__ double round_mul(double a, double b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+
+// The 8 corner values of the thread's tile points in one array (M^3 entries of
+// a batch entry); a null array of factors reads as 1.  The pointer is tested
+// once: a test per value puts every load behind the one before it.
+template <typename S, int NPT>
+__device__ __forceinline__ void load_points(const PipeP& p, const S* __restrict__ f, const int (&x)[NPT],
+                                            const int (&y)[NPT], int z, double (&v)[NPT][8]) {
+  if (f) {
+#pragma unroll
+    for (int k = 0; k < NPT; ++k)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[k][e] = (double)f[corner_index(p, x[k], y[k], z, e)];
+  } else {
+#pragma unroll
+    for (int k = 0; k < NPT; ++k)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[k][e] = 1.0;
+  }
+}
+
 template <typename TW>
 struct FoldTw {
   cx<TW> x, y, z;
@@ -306,20 +332,24 @@ __device__ void ph_fold_fftx(const PipeP& p, const PipeBufs& B, long item, int s
   const cx<double>* twM = static_cast<const cx<double>*>(B.twM);
   const int rs = H0 + 1;
   constexpr int NPT = TilePts<L0>::NPT;
-  T v[NPT][8];
   FoldTw<TW> ft[NPT];
+  int px[NPT], py[NPT];
 #pragma unroll
   for (int k = 0; k < NPT; ++k) {
     const int pt0 = threadIdx.x + k * kNT;
     const int pt = pt0 < H0 * YB ? pt0 : H0 * YB - 1;  // unconditional loads
-    const int x = pt % H0, y = y0 + pt / H0;
-    ft[k] = load_fold_tw<TW>(twM, x, y, z, p);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const long idx = corner_index(p, x, y, z, e);
-      v[k][e] = Eb ? (T)((double)fb[idx] * Eb[idx]) : fb[idx];
-    }
+    px[k] = pt % H0;
+    py[k] = y0 + pt / H0;
+    ft[k] = load_fold_tw<TW>(twM, px[k], py[k], z, p);
   }
+  double fv[NPT][8], ev[NPT][8];
+  load_points<T, NPT>(p, fb, px, py, z, fv);
+  load_points<double, NPT>(p, Eb, px, py, z, ev);
+  T v[NPT][8];
+#pragma unroll
+  for (int k = 0; k < NPT; ++k)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[k][e] = (T)round_mul(fv[k][e], ev[k][e]);
 #pragma unroll
   for (int k = 0; k < NPT; ++k) {
     const int pt = threadIdx.x + k * kNT;
@@ -749,15 +779,16 @@ __device__ void ph_ifftx_unfold(const PipeP& p, const PipeBufs& B, long item, in
   constexpr int NPT = TilePts<L0>::NPT;
   double ev[NPT][8];
   FoldTw<TW> ft[NPT];
+  int px[NPT], py[NPT];
 #pragma unroll
   for (int k = 0; k < NPT; ++k) {
     const int pt0 = threadIdx.x + k * kNT;
     const int pt = pt0 < H0 * YB ? pt0 : H0 * YB - 1;  // unconditional loads
-    const int x = pt % H0, y = y0 + pt / H0;
-    ft[k] = load_fold_tw<TW>(twM, x, y, z, p);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ev[k][e] = Eb ? Eb[corner_index(p, x, y, z, e)] : 1.0;
+    px[k] = pt % H0;
+    py[k] = y0 + pt / H0;
+    ft[k] = load_fold_tw<TW>(twM, px[k], py[k], z, p);
   }
+  load_points<double, NPT>(p, Eb, px, py, z, ev);
   tile_to_lds<T, L0>(p, static_cast<const cx<T>*>(B.ch), b, z, y0, lds);
   __syncthreads();
   lds_fft<T, TW, L0, +1>(lds, p.n_ch * YB, rs, 1);
@@ -772,7 +803,7 @@ __device__ void ph_ifftx_unfold(const PipeP& p, const PipeBufs& B, long item, in
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const T r = (T)((TW)v[e] * p.scale_unfold);
-      fb[corner_index(p, x, y, z, e)] = Eb ? (T)((double)r * ev[k][e]) : r;
+      fb[corner_index(p, x, y, z, e)] = (T)round_mul((double)r, ev[k][e]);
     }
   }
   __syncthreads();
@@ -884,20 +915,18 @@ __device__ void ph_unfold_fold(const PipeP& p, const PipeBufs& B, long item, int
   constexpr int NPT = TilePts<L0>::NPT;
   double eo[NPT][8], en[NPT][8];
   FoldTw<TW> ft[NPT];
-  const bool same_E = En == Eo;
+  int px[NPT], py[NPT];
 #pragma unroll
   for (int k = 0; k < NPT; ++k) {
     const int pt0 = threadIdx.x + k * kNT;
     const int pt = pt0 < H0 * YB ? pt0 : H0 * YB - 1;  // unconditional loads
-    const int x = pt % H0, y = y0 + pt / H0;
-    ft[k] = load_fold_tw<TW>(twM, x, y, z, p);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const long idx = corner_index(p, x, y, z, e);
-      eo[k][e] = Eo ? Eo[idx] : 1.0;
-      en[k][e] = same_E ? eo[k][e] : (En ? En[idx] : 1.0);
-    }
+    px[k] = pt % H0;
+    py[k] = y0 + pt / H0;
+    ft[k] = load_fold_tw<TW>(twM, px[k], py[k], z, p);
   }
+  load_points<double, NPT>(p, Eo, px, py, z, eo);
+  const bool other_E = En != Eo;
+  if (other_E) load_points<double, NPT>(p, En, px, py, z, en);
   // With one tile point per thread and 64 % H0 = 0 each wave's points are
   // whole tile rows; when the wave's groups can also take the x transforms of
   // those rows (every channel), the wave only ever touches its own LDS rows
@@ -920,14 +949,23 @@ __device__ void ph_unfold_fold(const PipeP& p, const PipeBufs& B, long item, int
     T v[8];
     gather_parities<T, TW>(p, lds, yy * rs + x, YB * rs, ft[k], v);
     wht8(v);
+    if (!other_E) {
+      // taken here, not where the loads are issued: a copy of eo into en's
+      // registers up there would wait for it
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        en[k][e] = eo[k][e];
+        asm volatile("" : "+v"(en[k][e]));
+      }
+    }
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       T r = (T)((TW)v[e] * p.scale_unfold);
-      if (Eo) r = (T)((double)r * eo[k][e]);
+      r = (T)round_mul((double)r, eo[k][e]);
       // a stored sweep's slice is read back only by the density pass, after
       // the sweep: a streaming store keeps it out of the caches the chain uses
       if constexpr (STORE) __builtin_nontemporal_store(r, fb + corner_index(p, x, y, z, e));
-      v[e] = En ? (T)((double)r * en[k][e]) : r;
+      v[e] = (T)round_mul((double)r, en[k][e]);
     }
     wht8(v);
     // the entries of this thread's point only: no barrier needed before reuse
