@@ -56,7 +56,7 @@ class MLP:
     def gradient(self, x, t):
         x = np.ascontiguousarray(x, dtype=np.float32).reshape(-1, self.dims[0])
         t = np.ascontiguousarray(t, dtype=np.float32).reshape(-1, self.dims[-1])
-        g = np.zeros(self.n_params, dtype=np.float32)
+        g = np.empty(self.n_params, dtype=np.float32)
         loss = C.c_double()
         L.check(L.lib().cfft_mlp_gradient(self._h, _fp(x), _fp(t), x.shape[0], C.byref(loss), _fp(g)))
         return float(loss.value), g

@@ -2,13 +2,14 @@
 // Adam) and inference on the GPU.  Weights are kept as an FP32 master copy for
 // the optimiser and a BF16 copy that feeds the matrix cores; every GEMM takes
 // BF16 operands (activations are rounded to BF16 when loaded) and accumulates
-// in FP32 with v_mfma_f32_16x16x16_bf16.  SiLU hidden activations, linear
+// in FP32 with v_mfma_f32_16x16x32_bf16.  SiLU hidden activations, linear
 // output, mean-squared-error loss.  No counterpart in the reference.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 #include <memory>
 #include <random>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/cfft_hip.h"
@@ -18,7 +19,8 @@ using namespace cfft;
 
 namespace {
 
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ inline uint16_t f2bf(float f) {
@@ -34,107 +36,247 @@ __device__ inline float dsilu(float z) {
   return s * (1.0f + z * (1.0f - s));
 }
 
-// Operand view: element (r, c) at p[r * rs + c * cs]; FP32 values are rounded
-// to BF16 on load, BF16 values are used as stored.
-struct OpF {
-  const float* p;
-  long rs, cs;
+// Operands of C(m, n) = sum_k A(m, k) B(k, n): x is the index that C keeps (m
+// or n), FP32 values are rounded to BF16 when loaded, BF16 values are used as
+// stored.  A lane's fragment is kf = 8 values of k at each of its TX indices.
+//   ContigK  element (x, k) at p[x * ld + k]: TX rows of 16, a lane reads 8
+//            neighbours along k
+//   StrideK  element (x, k) at p[k * ld + x]: a lane reads TX neighbours along
+//            x in each of its 8 rows, so its TX sub-tiles interleave and 16
+//            lanes cover 16 TX neighbours
+// Rows of C past the edge read the last valid one and are not stored; the
+// vector loads are aligned to an element only (any width, any offset).
+constexpr int kf = 8, kChunk = 32, kMaxWaves = 8;
+
+template <typename T, int TX>
+struct ContigK {
+  static constexpr int tx = TX;
+  using Elem = T;
+  const T* p;
+  long ld;
+  __device__ static int at(int x0, int i, int r, int) { return x0 + 16 * i + r; }
+  __device__ static bool own(int x0, int i, int r, int X) { return x0 + 16 * i + r < X; }
+  template <bool TAIL>
+  __device__ __forceinline__ void load(T (&v)[TX][kf], int x0, int r, int X, int k, int K) const {
+    typedef T Vec __attribute__((ext_vector_type(kf), aligned(sizeof(T))));
+#pragma unroll
+    for (int i = 0; i < TX; ++i) {
+      const T* q = p + (long)min(x0 + 16 * i + r, X - 1) * ld;
+      if constexpr (TAIL) {
+#pragma unroll
+        for (int j = 0; j < kf; ++j) {
+          const T u = q[min(k + j, K - 1)];
+          v[i][j] = k + j < K ? u : T(0);
+        }
+      } else {
+        const Vec u = *reinterpret_cast<const Vec*>(q + k);
+#pragma unroll
+        for (int j = 0; j < kf; ++j) v[i][j] = u[j];
+      }
+    }
+  }
 };
-struct OpB {
-  const uint16_t* p;
-  long rs, cs;
+
+template <typename T, int TX>
+struct StrideK {
+  static constexpr int tx = TX;
+  using Elem = T;
+  const T* p;
+  long ld;
+  // needs X >= TX: the last lane's neighbours start at X - TX at most
+  __device__ static int at(int x0, int i, int r, int X) { return min(x0 + TX * r, X - TX) + i; }
+  __device__ static bool own(int x0, int i, int r, int X) { return at(x0, i, r, X) >= x0 + TX * r; }
+  template <bool TAIL>
+  __device__ __forceinline__ void load(T (&v)[TX][kf], int x0, int r, int X, int k, int K) const {
+    typedef T Vec __attribute__((ext_vector_type(TX), aligned(sizeof(T))));
+    const T* q = p + min(x0 + TX * r, X - TX);
+#pragma unroll
+    for (int j = 0; j < kf; ++j) {
+      const Vec u = *reinterpret_cast<const Vec*>(q + (long)(TAIL ? min(k + j, K - 1) : k + j) * ld);
+#pragma unroll
+      for (int i = 0; i < TX; ++i) v[i][j] = !TAIL || k + j < K ? u[i] : T(0);
+    }
+  }
 };
-__device__ inline short ld(const OpF& o, int r, int c) { return (short)f2bf(o.p[r * o.rs + c * o.cs]); }
-__device__ inline short ld(const OpB& o, int r, int c) { return (short)o.p[r * o.rs + c * o.cs]; }
+
+__device__ __forceinline__ short to_bf(float v) { return (short)f2bf(v); }
+__device__ __forceinline__ short to_bf(uint16_t v) { return (short)v; }
+
+template <int TX, typename T>
+__device__ __forceinline__ void frag(s16x8 (&f)[TX], const T (&v)[TX][kf]) {
+#pragma unroll
+  for (int i = 0; i < TX; ++i) {
+#pragma unroll
+    for (int j = 0; j < kf; ++j) f[i][j] = to_bf(v[i][j]);
+  }
+}
 
 // Epilogues of C = A B (M x N):
-//   0 plain store                     out0 = C
-//   1 bias + SiLU                      out0 = Z = C + b, out1 = silu(Z)
-//   2 bias, linear                     out0 = C + b
-//   3 times SiLU'(Z) (backward)        out0 = C * silu'(aux)
-enum { EP_STORE = 0, EP_BIAS_SILU = 1, EP_BIAS = 2, EP_DSILU = 3 };
+//   GRAD       out0 = C (weight gradient); out1 = sum_k B(k, n) (bias gradient)
+//   BIAS_SILU  out0 = Z = C + b, out1 = silu(Z)
+//   BIAS       out0 = C + b
+//   MSE        Y = C + b, out0 = 2 (Y - aux) * scale; part[block] = sum (Y - aux)^2
+//   DSILU      out0 = C * silu'(aux) (backward)
+enum { EP_GRAD, EP_BIAS_SILU, EP_BIAS, EP_MSE, EP_DSILU };
 
 struct Ep {
-  int kind;
   float* out0;
   float* out1;
   const float* bias;  // N
-  const float* aux;   // M x N, row-major (EP_DSILU)
-  long ldo;           // row stride of out0 / out1 / aux
+  const float* aux;   // M x N, row-major
+  double* part;
+  long ldo;  // row stride of out0 / out1 / aux
+  float scale;
 };
 
-// One wavefront per 16 x 16 output tile; the K loop runs in steps of 16 with
-// one MFMA each.  Lane l holds A(row l%16, k 4(l/16)+j), B(k 4(l/16)+j, col
-// l%16) and D(row 4(l/16)+j, col l%16), j < 4.  Out-of-range rows, columns
-// and k are fed as zeros.
-template <typename TA, typename TB>
-__global__ void __launch_bounds__(256) k_gemm(TA A, TB B, int M, int N, int K, Ep ep) {
+// One workgroup per tile of 16 TM x 16 TN; its waves take the chunks of 32
+// along k in turn, one v_mfma_f32_16x16x32_bf16 per sub-tile and chunk, and
+// their partial tiles are added in LDS in wave order.  A batch of tens of rows
+// against layers of hundreds leaves some hundred tiles, so the time is one
+// chain of loads: splitting k keeps that chain at two chunks for K = 512, and
+// each lane's loads are vectors without a branch.  64 rows, 512 x 512 layer:
+// 27 -> 4.1 us (one wave per tile and 2-byte loads in one chain over k before),
+// weight gradient with its column sums 42 -> 5.0 us.  An empty kernel takes 2.
+// Lane l of the MFMA holds A(row l%16, k 8(l/16)+j), B(k 8(l/16)+j, col l%16),
+// j < 8, and D(row 4(l/16)+j, col l%16), j < 4.
+struct Shape {
+  int M, N, K;
+};
+
+template <int T>
+struct GemmLds {
+  float red[kMaxWaves][T][4][64];
+  float csum[kMaxWaves][2][16];
+  double lsum[kMaxWaves];
+};
+
+template <int EP, typename OA, typename OB, int T>
+__device__ __forceinline__ void gemm_tile(const OA& A, const OB& B, const Shape& sh, const Ep& ep, unsigned tile,
+                                          GemmLds<T>& lds) {
+  constexpr int TM = OA::tx, TN = OB::tx;
+  static_assert(TM * TN <= T && TN <= 2, "sub-tiles");
+  auto& red = lds.red;
+  auto& csum = lds.csum;
+  auto& lsum = lds.lsum;
+  const int M = sh.M, N = sh.N, K = sh.K;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int tiles_n = (N + 15) / 16;
-  const long tile = (long)blockIdx.x * 4 + wave;
-  if (tile >= (long)((M + 15) / 16) * tiles_n) return;
-  const int m0 = (int)(tile / tiles_n) * 16, n0 = (int)(tile % tiles_n) * 16;
-  const int r = lane & 15, kq = (lane >> 4) * 4;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    bf16x4 a, b;
+  const int nw = min((int)(blockDim.x >> 6), (K + kChunk - 1) / kChunk);  // waves with a chunk
+  const int tiles_n = (N + 16 * TN - 1) / (16 * TN);
+  const int m0 = (int)(tile / tiles_n) * 16 * TM, n0 = (int)(tile % tiles_n) * 16 * TN;
+  const int r = lane & 15, kl = (lane >> 4) * kf;
+  const bool sum_b = EP == EP_GRAD && m0 == 0;
+  f32x4 acc[TM][TN] = {};
+  float cs[TN] = {};
+  auto chunk = [&](auto tail, int k0) {
+    typename OA::Elem va[TM][kf];
+    typename OB::Elem vb[TN][kf];
+    A.template load<decltype(tail)::value>(va, m0, r, M, k0 + kl, K);
+    B.template load<decltype(tail)::value>(vb, n0, r, N, k0 + kl, K);
+    if constexpr (EP == EP_GRAD) {
+      if (sum_b) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int k = k0 + kq + j;
-      a[j] = (m0 + r < M && k < K) ? ld(A, m0 + r, k) : (short)0;
-      b[j] = (n0 + r < N && k < K) ? ld(B, k, n0 + r) : (short)0;
-    }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-  }
-  const int col = n0 + r;
-  if (col >= N) return;
+        for (int i = 0; i < TN; ++i) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int row = m0 + kq + j;
-    if (row >= M) continue;
-    const long o = (long)row * ep.ldo + col;
-    float v = acc[j];
-    switch (ep.kind) {
-      case EP_STORE: ep.out0[o] = v; break;
-      case EP_BIAS_SILU:
-        v += ep.bias[col];
-        ep.out0[o] = v;
-        ep.out1[o] = silu(v);
-        break;
-      case EP_BIAS: ep.out0[o] = v + ep.bias[col]; break;
-      default: ep.out0[o] = v * dsilu(ep.aux[o]); break;
+          for (int j = 0; j < kf; ++j) cs[i] += vb[i][j];
+        }
+      }
+    }
+    s16x8 a[TM], b[TN];
+    frag(a, va);
+    frag(b, vb);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[i]),
+                                                            __builtin_bit_cast(bf16x8, b[j]), acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  const int full = K / kChunk;
+  if (wave < nw) {
+#pragma unroll 2
+    for (int c = wave; c < full; c += nw) chunk(std::false_type{}, c * kChunk);
+    if (full * kChunk < K && full % nw == wave) chunk(std::true_type{}, full * kChunk);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) red[wave][i * TN + j][q][lane] = acc[i][j][q];
+      }
     }
   }
-}
-
-// Loss and output gradient: dY = 2 (Y - T) / (n_out * rows); partial sums of
-// (Y - T)^2 per block.
-__global__ void __launch_bounds__(256) k_mse(const float* __restrict__ Y, const float* __restrict__ T,
-                                             float* __restrict__ dY, long n, float scale,
-                                             double* __restrict__ part) {
-  __shared__ double red[256];
-  double acc = 0.0;
-  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-    const float d = Y[i] - T[i];
-    dY[i] = 2.0f * d * scale;
-    acc += (double)d * d;
+  if constexpr (EP == EP_GRAD) {
+    if (sum_b && wave < nw) {
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        cs[i] += __shfl_xor(cs[i], 16);
+        cs[i] += __shfl_xor(cs[i], 32);
+        if (lane < 16) csum[wave][i][lane] = cs[i];
+      }
+    }
   }
-  red[threadIdx.x] = acc;
   __syncthreads();
-  for (unsigned s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
+  double loss = 0.0;
+  for (int e = threadIdx.x; e < 256 * TM * TN; e += blockDim.x) {
+    const int t = e >> 8, q = (e >> 6) & 3, rm = 4 * ((e & 63) >> 4) + q, rn = e & 15;
+    float v = 0.f;
+    for (int w = 0; w < nw; ++w) v += red[w][t][q][e & 63];
+    if (!OA::own(m0, t / TN, rm, M) || !OB::own(n0, t % TN, rn, N)) continue;
+    const int row = OA::at(m0, t / TN, rm, M), col = OB::at(n0, t % TN, rn, N);
+    const long o = (long)row * ep.ldo + col;
+    if constexpr (EP == EP_GRAD) {
+      ep.out0[o] = v;
+    } else if constexpr (EP == EP_DSILU) {
+      ep.out0[o] = v * dsilu(ep.aux[o]);
+    } else {
+      v += ep.bias[col];
+      if constexpr (EP == EP_MSE) {
+        const float d = v - ep.aux[o];
+        ep.out0[o] = 2.0f * d * ep.scale;
+        loss += (double)d * d;
+      } else {
+        ep.out0[o] = v;
+        if constexpr (EP == EP_BIAS_SILU) ep.out1[o] = silu(v);
+      }
+    }
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+  if constexpr (EP == EP_GRAD) {
+    if (sum_b) {
+      for (int e = threadIdx.x; e < 16 * TN; e += blockDim.x) {
+        float v = 0.f;
+        for (int w = 0; w < nw; ++w) v += csum[w][e >> 4][e & 15];
+        if (OB::own(n0, e >> 4, e & 15, N)) ep.out1[OB::at(n0, e >> 4, e & 15, N)] = v;
+      }
+    }
+  }
+  if constexpr (EP == EP_MSE) {
+    for (int d = 1; d < 64; d <<= 1) loss += __shfl_xor(loss, d);
+    if (lane == 0) lsum[wave] = loss;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int w = 1; w < (int)(blockDim.x >> 6); ++w) loss += lsum[w];
+      ep.part[tile] = loss;
+    }
+  }
 }
 
-// Column sums of a rows x cols row-major matrix (bias gradients).
-__global__ void k_colsum(const float* __restrict__ X, float* __restrict__ out, int rows, int cols) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
-  float s = 0.f;
-  for (int r = 0; r < rows; ++r) s += X[(long)r * cols + c];
-  out[c] = s;
+template <int EP, typename OA, typename OB>
+__global__ void __launch_bounds__(64 * kMaxWaves) k_gemm(OA A, OB B, Shape sh, Ep ep) {
+  __shared__ GemmLds<OA::tx * OB::tx> lds;
+  gemm_tile<EP>(A, B, sh, ep, blockIdx.x, lds);
+}
+
+// Backward of one layer, both products in one launch (they only share dZ): the
+// first `n_w` workgroups take tiles of the weight gradient, the others those of
+// the input's gradient.
+template <typename OW, typename OD>
+__global__ void __launch_bounds__(64 * kMaxWaves) k_back(OW in, OW dz, Shape shw, Ep epw, unsigned n_w,
+                                                         ContigK<float, 1> dzk, OD w, Shape shd, Ep epd) {
+  __shared__ GemmLds<OW::tx * OW::tx> lds;
+  if (blockIdx.x < n_w) gemm_tile<EP_GRAD>(in, dz, shw, epw, blockIdx.x, lds);
+  else gemm_tile<EP_DSILU>(dzk, w, shd, epd, blockIdx.x - n_w, lds);
 }
 
 // Adam on the FP32 master parameters; refreshes the BF16 copy.
@@ -158,6 +300,17 @@ __global__ void k_to_bf16(const float* __restrict__ w, uint16_t* __restrict__ wb
   if (i < n) wb[i] = f2bf(w[i]);
 }
 
+// Device words into mapped host memory, four per thread as 16-byte stores.
+__global__ void __launch_bounds__(256) k_words(const float* __restrict__ src, float* __restrict__ dst, long n) {
+  const long i = 4 * (blockIdx.x * 256L + threadIdx.x);
+  typedef float Vec __attribute__((ext_vector_type(4), aligned(4)));
+  if (i + 4 <= n) {
+    *reinterpret_cast<f32x4*>(dst + i) = *reinterpret_cast<const Vec*>(src + i);
+  } else {
+    for (long j = i; j < n; ++j) dst[j] = src[j];
+  }
+}
+
 __global__ void k_gather_rows(const float* __restrict__ src, const int* __restrict__ idx, float* __restrict__ dst,
                               int rows, int cols) {
   const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
@@ -165,6 +318,32 @@ __global__ void k_gather_rows(const float* __restrict__ src, const int* __restri
   const int r = (int)(i / cols), c = (int)(i % cols);
   dst[i] = src[(long)idx[r] * cols + c];
 }
+
+}  // namespace
+
+namespace {
+
+long tiles(long n, int w) { return (n + w - 1) / w; }
+
+// Page-locked host memory.  Copies of the caller's pageable arrays go through
+// it in pieces, written by a kernel: 2.6 MB of gradients take 110 us this way
+// (one piece copied to the caller while the next is written), 220 us as an
+// asynchronous copy of the runtime.  Pieces of 256 KiB, 512 KiB and 1 MiB
+// measured 207, 178 and 224 us for the whole gradient call.
+struct HostBuf {
+  void* p = nullptr;
+  void alloc(size_t n) {
+    release();
+    hip_check(hipHostMalloc(&p, n, hipHostMallocDefault), "hipHostMalloc");
+  }
+  void release() {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+  }
+  ~HostBuf() { release(); }
+};
+constexpr int kSlots = 4;
+constexpr size_t kSlot = 512 << 10;
 
 }  // namespace
 
@@ -177,12 +356,17 @@ struct cfft_mlp {
   DevBuf w, wb, g, m, v;     // FP32 master, BF16 copy, gradient, Adam moments
   DevBuf Z, H;               // per layer pre/post activations (max_rows x dims[l+1])
   DevBuf dA, dB;             // backward ping-pong (max_rows x max dim)
-  DevBuf X, T, idx, xb, tb, part;
+  DevBuf X, T, xt;           // training set; the batch's inputs, then its targets
+  HostBuf part;              // squared error per tile of the output layer, written by the kernel
+  HostBuf stage;             // kSlots pieces of kSlot bytes between the caller's arrays and the device
+  hipEvent_t slot_done[kSlots] = {};
   long n_data = 0;
   long step = 0;
   hipStream_t stream = nullptr;
   std::vector<long> zoff;
   ~cfft_mlp() {
+    for (hipEvent_t e : slot_done)
+      if (e) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };
@@ -205,17 +389,8 @@ void ensure_rows(cfft_mlp* p, int rows) {
   for (int d : p->dims) dmax = std::max(dmax, d);
   p->dA.alloc(4L * rows * dmax);
   p->dB.alloc(4L * rows * dmax);
-  p->xb.alloc(4L * rows * p->dims[0]);
-  p->tb.alloc(4L * rows * p->dims[p->L]);
-  p->idx.alloc(4L * rows);
-}
-
-template <typename TA, typename TB>
-void gemm(cfft_mlp* p, TA A, TB B, int M, int N, int K, Ep ep) {
-  const long tiles = (long)((M + 15) / 16) * ((N + 15) / 16);
-  hipLaunchKernelGGL((k_gemm<TA, TB>), dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, p->stream, A, B, M, N, K,
-                     ep);
-  hip_check(hipGetLastError(), "k_gemm");
+  p->xt.alloc(4L * rows * (p->dims[0] + p->dims[p->L]));
+  p->part.alloc(8L * tiles(rows, 16) * tiles(p->dims[p->L], 16));
 }
 
 float* Zl(cfft_mlp* p, int l) { return static_cast<float*>(p->Z.p) + p->zoff[l]; }
@@ -223,65 +398,139 @@ float* Hl(cfft_mlp* p, int l) { return static_cast<float*>(p->H.p) + p->zoff[l];
 const uint16_t* Wb(cfft_mlp* p, int l) { return static_cast<const uint16_t*>(p->wb.p) + p->woff[l]; }
 const float* Bias(cfft_mlp* p, int l) { return static_cast<const float*>(p->w.p) + p->boff[l]; }
 
+// Launches one GEMM; returns its workgroup count.
+template <int EP, typename OA, typename OB>
+int gemm(cfft_mlp* p, OA A, OB B, int M, int N, int K, const Ep& ep) {
+  const long grid = tiles(M, 16 * OA::tx) * tiles(N, 16 * OB::tx);
+  const int waves = (int)std::min<long>(kMaxWaves, tiles(K, kChunk));
+  hipLaunchKernelGGL((k_gemm<EP, OA, OB>), dim3((unsigned)grid), dim3(64 * waves), 0, p->stream, A, B,
+                     Shape{M, N, K}, ep);
+  hip_check(hipGetLastError(), "k_gemm");
+  return (int)grid;
+}
+
+// Both products of layer l's backward: dW_l = in^T dZ (K x N) with db_l = column
+// sums of dZ, and dZ_{l-1} = (dZ_l W_l^T) * silu'(Z_{l-1}) (rows x K) unless l = 0.
+template <int TX>
+void back(cfft_mlp* p, int l, const float* in, const float* dz, float* dz_in, int rows) {
+  const int K = p->dims[l], N = p->dims[l + 1];
+  float* g = static_cast<float*>(p->g.p);
+  const StrideK<float, TX> A{in, K}, B{dz, N};
+  Ep ew{};
+  ew.out0 = g + p->woff[l];
+  ew.out1 = g + p->boff[l];
+  ew.ldo = N;
+  if (l == 0) {
+    gemm<EP_GRAD>(p, A, B, K, N, rows, ew);
+    return;
+  }
+  Ep ed{};
+  ed.out0 = dz_in;
+  ed.aux = Zl(p, l - 1);
+  ed.ldo = K;
+  const ContigK<float, 1> D{dz, N};
+  const ContigK<uint16_t, 1> W{Wb(p, l), N};
+  const long nw = tiles(K, 16 * TX) * tiles(N, 16 * TX), nd = tiles(rows, 16) * tiles(K, 16);
+  const int waves = (int)std::min<long>(kMaxWaves, tiles(std::max(rows, N), kChunk));
+  hipLaunchKernelGGL((k_back<StrideK<float, TX>, ContigK<uint16_t, 1>>), dim3((unsigned)(nw + nd)), dim3(64 * waves),
+                     0, p->stream, A, B, Shape{K, N, rows}, ew, (unsigned)nw, D, W, Shape{rows, K, N}, ed);
+  hip_check(hipGetLastError(), "k_back");
+}
+
+// Enqueues the caller's array `src` to the device, through the staging pieces
+// at byte `at` where it fits (the stream is idle when a call begins).
+void copy_in(cfft_mlp* p, void* dst, const void* src, size_t bytes, size_t at) {
+  if (at + bytes <= kSlots * kSlot) {
+    char* h = static_cast<char*>(p->stage.p) + at;
+    std::memcpy(h, src, bytes);
+    src = h;
+  }
+  hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, p->stream), "H2D");
+}
+
+// Device array to the caller's, through the staging pieces in turn; the stream's
+// work is done on return.
+void copy_out(cfft_mlp* p, float* dst, const void* src, size_t bytes) {
+  const size_t n = (bytes + kSlot - 1) / kSlot;
+  auto part = [&](size_t i) { return std::min(kSlot, bytes - i * kSlot); };
+  auto slot = [&](size_t i) { return static_cast<float*>(p->stage.p) + (i % kSlots) * (kSlot / 4); };
+  auto fetch = [&](size_t i) {
+    const long words = (long)part(i) / 4;
+    hipLaunchKernelGGL(k_words, dim3(nblk(words, 1024)), dim3(256), 0, p->stream,
+                       static_cast<const float*>(src) + i * (kSlot / 4), slot(i), words);
+    hip_check(hipGetLastError(), "k_words");
+    hip_check(hipEventRecord(p->slot_done[i % kSlots], p->stream), "hipEventRecord");
+  };
+  for (size_t i = 0; i < std::min<size_t>(n, kSlots); ++i) fetch(i);
+  for (size_t i = 0; i < n; ++i) {
+    hip_check(hipEventSynchronize(p->slot_done[i % kSlots]), "hipEventSynchronize");
+    std::memcpy(dst + i * (kSlot / 4), slot(i), part(i));
+    if (i + kSlots < n) fetch(i + kSlots);
+  }
+}
+
+// Layer l on `rows` inputs at `in`; W of layer l is K x N row-major.
+template <int EP>
+int layer(cfft_mlp* p, int l, const float* in, int rows, Ep ep) {
+  const int K = p->dims[l], N = p->dims[l + 1];
+  ep.bias = Bias(p, l);
+  ep.ldo = N;
+  const ContigK<float, 1> A{in, K};
+  return N >= 2 ? gemm<EP>(p, A, StrideK<uint16_t, 2>{Wb(p, l), N}, rows, N, K, ep)
+                : gemm<EP>(p, A, StrideK<uint16_t, 1>{Wb(p, l), N}, rows, N, K, ep);
+}
+
+// The hidden layers on `rows` inputs at x; returns the last layer's input.
+const float* hidden(cfft_mlp* p, const float* x, int rows) {
+  const float* in = x;
+  for (int l = 0; l + 1 < p->L; ++l) {
+    Ep ep{};
+    ep.out0 = Zl(p, l);
+    ep.out1 = Hl(p, l);
+    layer<EP_BIAS_SILU>(p, l, in, rows, ep);
+    in = Hl(p, l);
+  }
+  return in;
+}
+
 // Forward on `rows` inputs at x (device, rows x dims[0]); the output is Z of
 // the last layer.
 void forward(cfft_mlp* p, const float* x, int rows) {
-  const float* in = x;
-  for (int l = 0; l < p->L; ++l) {
-    const int K = p->dims[l], N = p->dims[l + 1];
-    Ep ep{};
-    ep.kind = l + 1 < p->L ? EP_BIAS_SILU : EP_BIAS;
-    ep.out0 = Zl(p, l);
-    ep.out1 = Hl(p, l);
-    ep.bias = Bias(p, l);
-    ep.ldo = N;
-    // W of layer l is K x N row-major
-    gemm(p, OpF{in, K, 1}, OpB{Wb(p, l), N, 1}, rows, N, K, ep);
-    in = Hl(p, l);
-  }
+  Ep ep{};
+  ep.out0 = Zl(p, p->L - 1);
+  layer<EP_BIAS>(p, p->L - 1, hidden(p, x, rows), rows, ep);
+}
+
+// Forward against the targets t: dY at dA and the squared errors per tile in
+// `part`; returns their count.
+int forward_loss(cfft_mlp* p, const float* x, const float* t, int rows) {
+  Ep ep{};
+  ep.out0 = static_cast<float*>(p->dA.p);
+  ep.aux = t;
+  ep.part = static_cast<double*>(p->part.p);
+  ep.scale = 1.0f / (float)((long)rows * p->dims[p->L]);
+  return layer<EP_MSE>(p, p->L - 1, hidden(p, x, rows), rows, ep);
 }
 
 // Backward from dY (rows x dims[L]) at dA; fills the gradient buffer.
 void backward(cfft_mlp* p, const float* x, int rows) {
-  float* g = static_cast<float*>(p->g.p);
   float* cur = static_cast<float*>(p->dA.p);  // dZ of layer l
   float* nxt = static_cast<float*>(p->dB.p);
   for (int l = p->L - 1; l >= 0; --l) {
-    const int K = p->dims[l], N = p->dims[l + 1];
     const float* in = l == 0 ? x : Hl(p, l - 1);
-    // dW_l = in^T dZ  (K x N)
-    Ep ew{};
-    ew.kind = EP_STORE;
-    ew.out0 = g + p->woff[l];
-    ew.ldo = N;
-    gemm(p, OpF{in, 1, K}, OpF{cur, N, 1}, K, N, rows, ew);
-    hipLaunchKernelGGL(k_colsum, dim3(nblk(N, 256)), dim3(256), 0, p->stream, cur, g + p->boff[l], rows, N);
-    hip_check(hipGetLastError(), "k_colsum");
-    if (l == 0) break;
-    // dZ_{l-1} = (dZ_l W_l^T) * silu'(Z_{l-1})   (rows x K)
-    Ep ed{};
-    ed.kind = EP_DSILU;
-    ed.out0 = nxt;
-    ed.aux = Zl(p, l - 1);
-    ed.ldo = K;
-    gemm(p, OpF{cur, N, 1}, OpB{Wb(p, l), 1, N}, rows, K, N, ed);
+    if (p->dims[l] >= 2 && p->dims[l + 1] >= 2) back<2>(p, l, in, cur, nxt, rows);
+    else back<1>(p, l, in, cur, nxt, rows);
     std::swap(cur, nxt);
   }
 }
 
-double loss_grad(cfft_mlp* p, const float* t, int rows) {
-  const int out = p->dims[p->L];
-  const long n = (long)rows * out;
-  const unsigned nb = (unsigned)std::min<long>(256, std::max<long>(1, nblk(n, 256)));
-  hipLaunchKernelGGL(k_mse, dim3(nb), dim3(256), 0, p->stream, Zl(p, p->L - 1), t,
-                     static_cast<float*>(p->dA.p), n, 1.0f / (float)n, static_cast<double*>(p->part.p));
-  hip_check(hipGetLastError(), "k_mse");
-  std::vector<double> h(nb);
-  hip_check(hipMemcpyAsync(h.data(), p->part.p, 8 * nb, hipMemcpyDeviceToHost, p->stream), "D2H");
-  hip_check(hipStreamSynchronize(p->stream), "sync");
+// Mean squared error from the `parts` tile sums of forward_loss, once the
+// stream is idle.
+double mean_loss(const cfft_mlp* p, int parts, int rows) {
+  const double* h = static_cast<const double*>(p->part.p);
   double s = 0.0;
-  for (double v : h) s += v;
-  return s / (double)n;
+  for (int i = 0; i < parts; ++i) s += h[i];
+  return s / (double)((long)rows * p->dims[p->L]);
 }
 
 }  // namespace
@@ -308,6 +557,10 @@ int cfft_mlp_create(int32_t n_layers, const int32_t* dims, uint64_t seed, cfft_m
     }
     p->n_params = off;
     hip_check(hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking), "hipStreamCreate");
+    for (hipEvent_t& e : p->slot_done) {
+      hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+    }
+    p->stage.alloc(kSlots * kSlot);
     // He-style initialisation (normal, std sqrt(2 / fan_in)), zero biases
     std::vector<float> w(p->n_params, 0.f);
     std::mt19937_64 rng(seed);
@@ -320,7 +573,6 @@ int cfft_mlp_create(int32_t n_layers, const int32_t* dims, uint64_t seed, cfft_m
     p->g.alloc(4 * p->n_params);
     p->m.alloc(4 * p->n_params);
     p->v.alloc(4 * p->n_params);
-    p->part.alloc(8 * 256);
     hip_check(hipMemcpy(p->w.p, w.data(), 4 * p->n_params, hipMemcpyHostToDevice), "upload");
     hip_check(hipMemset(p->m.p, 0, 4 * p->n_params), "memset");
     hip_check(hipMemset(p->v.p, 0, 4 * p->n_params), "memset");
@@ -363,11 +615,9 @@ int cfft_mlp_forward(cfft_mlp* p, const float* x, int32_t rows, float* y) {
   return guarded([&] {
     require(p && x && y && rows >= 1, CFFT_ERR_INVALID, "bad argument");
     ensure_rows(p, rows);
-    hip_check(hipMemcpyAsync(p->xb.p, x, 4L * rows * p->dims[0], hipMemcpyHostToDevice, p->stream), "H2D");
-    forward(p, static_cast<const float*>(p->xb.p), rows);
-    hip_check(hipMemcpyAsync(y, Zl(p, p->L - 1), 4L * rows * p->dims[p->L], hipMemcpyDeviceToHost, p->stream),
-              "D2H");
-    hip_check(hipStreamSynchronize(p->stream), "sync");
+    copy_in(p, p->xt.p, x, 4L * rows * p->dims[0], 0);
+    forward(p, static_cast<const float*>(p->xt.p), rows);
+    copy_out(p, y, Zl(p, p->L - 1), 4L * rows * p->dims[p->L]);
   });
 }
 
@@ -375,16 +625,17 @@ int cfft_mlp_gradient(cfft_mlp* p, const float* x, const float* t, int32_t rows,
   return guarded([&] {
     require(p && x && t && rows >= 1, CFFT_ERR_INVALID, "bad argument");
     ensure_rows(p, rows);
-    hip_check(hipMemcpyAsync(p->xb.p, x, 4L * rows * p->dims[0], hipMemcpyHostToDevice, p->stream), "H2D");
-    hip_check(hipMemcpyAsync(p->tb.p, t, 4L * rows * p->dims[p->L], hipMemcpyHostToDevice, p->stream), "H2D");
-    forward(p, static_cast<const float*>(p->xb.p), rows);
-    const double l = loss_grad(p, static_cast<const float*>(p->tb.p), rows);
-    backward(p, static_cast<const float*>(p->xb.p), rows);
+    float* xb = static_cast<float*>(p->xt.p);
+    float* tb = xb + (long)rows * p->dims[0];
+    const size_t nx = 4L * rows * p->dims[0], nt = 4L * rows * p->dims[p->L];
+    copy_in(p, xb, x, nx, 0);
+    copy_in(p, tb, t, nt, nx);
+    const int parts = forward_loss(p, xb, tb, rows);
+    backward(p, xb, rows);
+    if (grad) copy_out(p, grad, p->g.p, 4 * p->n_params);
+    else hip_check(hipStreamSynchronize(p->stream), "sync");
+    const double l = mean_loss(p, parts, rows);
     if (loss) *loss = l;
-    if (grad) {
-      hip_check(hipMemcpyAsync(grad, p->g.p, 4 * p->n_params, hipMemcpyDeviceToHost, p->stream), "D2H");
-    }
-    hip_check(hipStreamSynchronize(p->stream), "sync");
   });
 }
 
@@ -413,16 +664,16 @@ int cfft_mlp_train(cfft_mlp* p, const float* X, const float* T, int64_t n, int32
       long seen = 0;
       for (long s0 = 0; s0 < n; s0 += batch) {
         const int rows = (int)std::min<long>(batch, n - s0);
+        float* xb = static_cast<float*>(p->xt.p);
+        float* tb = xb + (long)rows * din;
         const int* idx = static_cast<const int*>(perm_dev.p) + s0;
         hipLaunchKernelGGL(k_gather_rows, dim3(nblk((long)rows * din, 256)), dim3(256), 0, p->stream,
-                           static_cast<const float*>(p->X.p), idx, static_cast<float*>(p->xb.p), rows, din);
+                           static_cast<const float*>(p->X.p), idx, xb, rows, din);
         hipLaunchKernelGGL(k_gather_rows, dim3(nblk((long)rows * dout, 256)), dim3(256), 0, p->stream,
-                           static_cast<const float*>(p->T.p), idx, static_cast<float*>(p->tb.p), rows, dout);
+                           static_cast<const float*>(p->T.p), idx, tb, rows, dout);
         hip_check(hipGetLastError(), "k_gather_rows");
-        forward(p, static_cast<const float*>(p->xb.p), rows);
-        lsum += loss_grad(p, static_cast<const float*>(p->tb.p), rows) * rows;
-        seen += rows;
-        backward(p, static_cast<const float*>(p->xb.p), rows);
+        const int parts = forward_loss(p, xb, tb, rows);
+        backward(p, xb, rows);
         ++p->step;
         const float c1 = 1.f - std::pow(b1, (float)p->step), c2 = 1.f - std::pow(b2, (float)p->step);
         hipLaunchKernelGGL(k_adam, dim3(nblk(p->n_params, 256)), dim3(256), 0, p->stream,
@@ -430,6 +681,9 @@ int cfft_mlp_train(cfft_mlp* p, const float* X, const float* T, int64_t n, int32
                            static_cast<const float*>(p->g.p), static_cast<float*>(p->m.p),
                            static_cast<float*>(p->v.p), p->n_params, lr, b1, b2, eps, c1, c2);
         hip_check(hipGetLastError(), "k_adam");
+        hip_check(hipStreamSynchronize(p->stream), "sync");
+        lsum += mean_loss(p, parts, rows) * rows;
+        seen += rows;
       }
       if (loss_per_epoch) loss_per_epoch[ep] = lsum / (double)seen;
     }
