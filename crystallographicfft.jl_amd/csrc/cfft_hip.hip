@@ -442,9 +442,13 @@ void build_plan(cfft_plan* p, const int* N, const std::vector<Op>& ops, double d
   } else if (!is_q_path(p)) {
     ReverseLookup rl = reverse_lookup(p->spec, ops);
     std::vector<uint32_t> tab((size_t)8 * p->n_alive, 0xFFFFFu);
+    const bool cube = p->H[0] == p->H[1] && p->H[1] == p->H[2];
     for (long e = 0; e < p->n_alive; ++e) {
       int q[3];
       q_of(e, q);
+      // cubic grids: z fastest in a plane, the order that P4 reads
+      const long k = e % p->H3, yz = 1L * p->H[1] * p->H[2], k1 = k % p->H[1], k2 = (k % yz) / p->H[1];
+      const long row = cube ? e - k % yz + k1 * p->H[2] + k2 : e;
       for (int a = 0; a < p->d; ++a) {
         long h[3];
         for (int dd = 0; dd < 3; ++dd) h[dd] = q[dd] + 1L * p->M[dd] * alphas[a][dd];
@@ -452,7 +456,7 @@ void build_plan(cfft_plan* p, const int* N, const std::vector<Op>& ops, double d
         uint32_t ent = 0xFFFFFu;
         if (rl.idx[li] >= 0)
           ent = (uint32_t)rl.idx[li] | ((uint32_t)rl.j[li] << 20) | ((uint32_t)rl.conj[li] << 31);
-        tab[(size_t)e * 8 + a] = ent;
+        tab[(size_t)row * 8 + a] = ent;
       }
     }
     upload_bytes(p->d_btab, tab.data(), tab.size() * 4);
@@ -711,7 +715,10 @@ PipeP pipe_params(cfft_plan* p, const ESel& es) {
   pp.n_ch = p->n_ch;
   for (int c = 0; c < 8; ++c) pp.offs[c] = 0;
   for (int c = 0; c < p->n_ch; ++c) pp.offs[c] = p->offs[c][0] | (p->offs[c][1] << 1) | (p->offs[c][2] << 2);
-  for (int i = 0; i < 8; ++i) pp.chmap[i] = p->chmap[i];
+  for (int i = 0; i < 8; ++i) {
+    pp.chmap[i] = p->chmap[i];
+    pp.chbits |= (uint32_t)(p->chmap[i] >= 0 ? p->chmap[i] : 15) << (4 * i);
+  }
   pp.batch = p->batch;
   // y rows per tile: a power of two (shift/mask tile indexing), by default the
   // largest <= 8 dividing H1; n_ch * YB <= 64 rows fit the tile's LDS
@@ -842,7 +849,7 @@ void launch_p4(cfft_plan* p, const PipeP& pp, const PipeBufs& B, hipStream_t s) 
   StageTimer st(p, s, CFFT_STAGE_IRECON);
   const unsigned g = (unsigned)n_planes(p);
 #define CFFT_P4(L) \
-  case L: hipLaunchKernelGGL((k_p4<T, double, L, L>), dim3(g), dim3(kNT), 0, s, pp, B); break;
+  case L: hipLaunchKernelGGL((k_p4<T, double, L, L>), dim3(g), dim3(p4_threads(L * L)), 0, s, pp, B); break;
   CFFT_LEN_SWITCH(p->H[1], CFFT_P4)
 #undef CFFT_P4
   launch_check<T>("k_p4");

@@ -28,6 +28,7 @@ constexpr int kNT = 256;  // threads per workgroup of the phase kernels
 struct PipeP {
   int M[3], H[3];
   int n_ch, offs[8], chmap[8];
+  uint32_t chbits;  // chmap as nibbles, 15: extinct
   int batch, YB;  // y rows per P1/P5 tile: a power of two dividing H1
   int ybs;        // log2(YB)
   int n_spec, d, P, Pn[3];
@@ -53,7 +54,7 @@ struct PipeBufs {
   const double* K;    // kernel (nullptr: 1)
   const void* W;      // exp(2 pi i j / P)
   const void* twM;    // fold twiddles (M0 + M1 + M2)
-  const uint32_t* btab;  // inverse reconstruction table [e][8]
+  const uint32_t* btab;  // inverse reconstruction table [e][8] (cubic: the points of a plane z fastest)
   const void* grep;      // path QR: Q-multiplied values at the orbit representatives
   const uint32_t* qmap;  // path QR: element -> rep (bits 0-19) | phase exponent << 20
   const void* qsep;      // path QS: axis factors F[d][s][q] (cx<double>, 3 x 8 x M0)
@@ -437,14 +438,16 @@ __device__ __forceinline__ void ph_recon_point(const PipeP& p, const PipeBufs& B
   const int b = valid ? (int)(pt / p.n_spec) : 0;
   const int i = valid ? (int)(pt - (long)b * p.n_spec) : 0;
   cx<T> v = {T(0), T(0)};
+  // ahead of the gather that the sum waits for
+  const TW kk = B.K ? (TW)B.K[i] : TW(1);
   if (valid && a < p.d) {
     const int* hs = B.hs;
     const int h0 = hs[3 * i], h1 = hs[3 * i + 1], h2 = hs[3 * i + 2];
     const int q0 = pmodi(p.R[a][0] * h0 + p.R[a][3] * h1 + p.R[a][6] * h2, p.M[0]);
     const int q1 = pmodi(p.R[a][1] * h0 + p.R[a][4] * h1 + p.R[a][7] * h2, p.M[1]);
     const int q2 = pmodi(p.R[a][2] * h0 + p.R[a][5] * h1 + p.R[a][8] * h2, p.M[2]);
-    const int c = p.chmap[(q0 & 1) | ((q1 & 1) << 1) | ((q2 & 1) << 2)];
-    if (c >= 0) {
+    const int c = (p.chbits >> (4 * ((q0 & 1) | ((q1 & 1) << 1) | ((q2 & 1) << 2)))) & 15;
+    if (c != 15) {
       const int j = h0 * p.t[a][0] * p.Pn[0] + h1 * p.t[a][1] * p.Pn[1] + h2 * p.t[a][2] * p.Pn[2];
       const long H3 = (long)p.H[0] * p.H[1] * p.H[2];
       const long k = ((long)(q0 >> 1) * p.H[2] + (q2 >> 1)) * p.H[1] + (q1 >> 1);
@@ -455,17 +458,33 @@ __device__ __forceinline__ void ph_recon_point(const PipeP& p, const PipeBufs& B
   }
   v = octet_sum(v);
   if (valid && a == 0) {
-    const TW kk = B.K ? (TW)B.K[i] : TW(1);
     static_cast<cx<T>*>(B.F)[pt] = {(T)((TW)v.x * kk), (T)((TW)v.y * kk)};
   }
+}
+
+// c ? a : b on the components (a select of two array elements written as
+// `c ? arr[i] : arr[j]` can become a select of addresses, which moves the
+// array to scratch memory)
+template <typename U>
+__device__ __forceinline__ cx<U> csel(bool c, cx<U> a, cx<U> b) {
+  return {c ? a.x : b.x, c ? a.y : b.y};
 }
 
 // ---- P4: inverse reconstruction, IFFT z, IFFT y of one (b, c, x) plane ------
 // G0(q) = (1/d) sum_alpha F(q + M alpha) through the reverse-lookup table
 // (src/krfft.jl:1285-1311, src/centering_fold.jl:782-813).
-template <typename T, typename TW, int L1, int L2>
-__device__ void ph_irecon_ifft_zy(const PipeP& p, const PipeBufs& B, long item, cx<T>* lds) {
-  constexpr int rs = L1 + 1, NP = L1 * L2, NIT = (NP + kNT - 1) / kNT;
+// Bound by its chain of loads (table, then the gathers of the eight aliases)
+// and by the instructions of the sum, with few workgroups: the gathers of a
+// thread's points are in flight together, lanes run along z, where neighbours
+// (h3) lie together in the spectral list, the phases come from a copy of the P
+// phases in LDS (`wl`, of kPhases entries) where it fits, and a workgroup has
+// up to 512 threads.  Ia-3d 96^3 mixed, 2 fields: 8.9 -> 6.5 us (one gather
+// after the other, 256 threads before); Im-3m 128^3 FP64, 1 field: 7.9 -> 8.6 us
+// in the trace, the backward transform 12.96 -> 12.94 us.
+constexpr int kPhases = 512;
+template <typename T, typename TW, int L1, int L2, int NT>
+__device__ void ph_irecon_ifft_zy(const PipeP& p, const PipeBufs& B, long item, cx<T>* lds, cx<TW>* wl) {
+  constexpr int rs = L1 + 1, NP = L1 * L2, NIT = (NP + NT - 1) / NT;
   const long H3 = (long)p.H[0] * NP;
   const long n_alive = (long)p.n_ch * H3;
   const int b = (int)(item / ((long)p.n_ch * p.H[0]));
@@ -473,38 +492,71 @@ __device__ void ph_irecon_ifft_zy(const PipeP& p, const PipeBufs& B, long item, 
   const cx<T>* Fb = static_cast<const cx<T>*>(B.F) + (long)b * p.n_spec;
   const cx<TW>* W = static_cast<const cx<TW>*>(B.W);
   const uint4* tab4 = reinterpret_cast<const uint4*>(B.btab);
-  // all table rows of this thread first, then the gathers
+  // all table rows of this thread first, then the gathers of GRP points at a
+  // time; rows past the plane are extinct
   uint4 ta[NIT], tb[NIT];
 #pragma unroll
   for (int it = 0; it < NIT; ++it) {
-    const int i = threadIdx.x + it * kNT;
+    const int i = threadIdx.x + it * NT;
+    ta[it] = tb[it] = {~0u, ~0u, ~0u, ~0u};
     if (i < NP) {
       ta[it] = tab4[2 * (e0 + i)];
       tb[it] = tab4[2 * (e0 + i) + 1];
     }
   }
+  constexpr int GRP = NIT % 4 == 0 ? 4 : (NIT % 3 == 0 ? 3 : (NIT % 2 == 0 ? 2 : 1));
+  auto gather = [&](const cx<TW>* w) {
 #pragma unroll
-  for (int it = 0; it < NIT; ++it) {
-    const int i = threadIdx.x + it * kNT;
-    if (i >= NP) continue;
-    const uint32_t ent[8] = {ta[it].x, ta[it].y, ta[it].z, ta[it].w, tb[it].x, tb[it].y, tb[it].z, tb[it].w};
-    cx<T> acc = {T(0), T(0)};
+    for (int i0 = 0; i0 < NIT; i0 += GRP) {
+      cx<T> f[GRP][8];
 #pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      const uint32_t idx = ent[a] & 0xFFFFFu;
-      const bool ok = idx != 0xFFFFFu;
-      cx<T> f = Fb[ok ? idx : 0];
-      if (ent[a] >> 31) f.y = -f.y;
-      const cx<T> prod = twmul<T, TW, -1>(f, W[(ent[a] >> 20) & 0x7FFu]);
-      if (ok) acc = cadd(acc, prod);
+      for (int g = 0; g < GRP; ++g) {
+        const uint4 u = ta[i0 + g], v = tb[i0 + g];
+        const uint32_t ent[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int a = 0; a < 8; ++a) {
+          const uint32_t idx = ent[a] & 0xFFFFFu;
+          f[g][a] = Fb[idx != 0xFFFFFu ? idx : 0];
+        }
+      }
+      // keeps the loads here, together: sunk into a test of each alias they
+      // would wait for one another
+#pragma unroll
+      for (int g = 0; g < GRP; ++g) {
+#pragma unroll
+        for (int a = 0; a < 8; ++a) asm volatile("" : "+v"(f[g][a].x), "+v"(f[g][a].y));
+      }
+#pragma unroll
+      for (int g = 0; g < GRP; ++g) {
+        const int i = threadIdx.x + (i0 + g) * NT;
+        const uint4 u = ta[i0 + g], v = tb[i0 + g];
+        const uint32_t ent[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+        cx<T> acc = {T(0), T(0)};
+#pragma unroll
+        for (int a = 0; a < 8; ++a) {
+          const bool ok = (ent[a] & 0xFFFFFu) != 0xFFFFFu;
+          cx<T> fa = f[g][a];
+          if (ent[a] >> 31) fa.y = -fa.y;
+          const cx<T> prod = twmul<T, TW, -1>(fa, w[ok ? (ent[a] >> 20) & 0x7FFu : 0u]);
+          acc = cadd(acc, csel(ok, prod, {T(0), T(0)}));
+        }
+        if (i < NP)
+          lds[(i % L2) * rs + i / L2] = {(T)((TW)acc.x * p.scale_irecon), (T)((TW)acc.y * p.scale_irecon)};
+      }
     }
-    lds[(i / L1) * rs + (i % L1)] = {(T)((TW)acc.x * p.scale_irecon), (T)((TW)acc.y * p.scale_irecon)};
+  };
+  if (p.P <= kPhases) {
+    for (int i = threadIdx.x; i < p.P; i += NT) wl[i] = W[i];
+    __syncthreads();
+    gather(wl);
+  } else {
+    gather(W);
   }
   __syncthreads();
-  lds_fft<T, TW, L2, +1>(lds, L1, 1, rs);
+  lds_fft<T, TW, L2, +1, NT>(lds, L1, 1, rs);
   {  // IFFT y, each row stored straight from its transform lanes
     cx<T>* plane = static_cast<cx<T>*>(B.ch) + item * (long)NP;
-    rows_fft_to_global<T, TW, L1, +1, kNT, L2>(lds, plane, plane, L2);
+    rows_fft_to_global<T, TW, L1, +1, NT, L2>(lds, plane, plane, L2);
   }
   __syncthreads();
 }
@@ -547,14 +599,6 @@ __device__ void ph_expand_ifft_zy(const PipeP& p, const PipeBufs& B, long item, 
 // off = 0 the two self-paired lines 0 and L/2 share unit 0; for odd L the one
 // self-paired line is its own unit (a = b).  Units 0 .. (L + 1) / 2 - 1 cover
 // every line once.
-// c ? a : b on the components (a select of two array elements written as
-// `c ? arr[i] : arr[j]` can become a select of addresses, which moves the
-// array to scratch memory)
-template <typename U>
-__device__ __forceinline__ cx<U> csel(bool c, cx<U> a, cx<U> b) {
-  return {c ? a.x : b.x, c ? a.y : b.y};
-}
-
 template <int L>
 __device__ __forceinline__ void unit_lines(int u, int off, int& a, int& b, bool& pair) {
   if (off == 0) {
@@ -1001,10 +1045,17 @@ __global__ void __launch_bounds__(kNT) k_p3(PipeP p, PipeBufs B) {
   ph_recon_point<T, TW>(p, B, pt, pt < (long)p.n_spec * p.batch);
 }
 
+// Threads of a P4 workgroup: the points of a plane in as few rounds as 512
+// threads allow, in whole waves.
+constexpr int p4_threads(int np) {
+  const int rounds = (np + 511) / 512;
+  return ((np + rounds - 1) / rounds + 63) / 64 * 64;
+}
 template <typename T, typename TW, int L1, int L2>
-__global__ void __launch_bounds__(kNT) k_p4(PipeP p, PipeBufs B) {
+__global__ void __launch_bounds__(p4_threads(L1 * L2)) k_p4(PipeP p, PipeBufs B) {
   __shared__ cx<T> lds[L2 * (L1 + 1)];
-  ph_irecon_ifft_zy<T, TW, L1, L2>(p, B, blockIdx.x, lds);
+  __shared__ cx<TW> wl[kPhases];
+  ph_irecon_ifft_zy<T, TW, L1, L2, p4_threads(L1 * L2)>(p, B, blockIdx.x, lds, wl);
 }
 
 template <typename T, typename TW, int L1, int L2>
@@ -1120,6 +1171,7 @@ __global__ void __launch_bounds__(kNT) k_sweep(PipeP p, PipeBufs B, int step0, i
   constexpr int TILE = 64 * (L + 1);
   constexpr int PLANE = L * (L + 1);
   __shared__ cx<T> lds[TILE > PLANE ? TILE : PLANE];
+  __shared__ cx<TW> wl[kPhases];
   const long n_tiles = (long)p.batch * p.H[2] * (p.H[1] / p.YB);
   const long n_planes = (long)p.batch * p.n_ch * p.H[0];
   const long n_pts = (long)p.n_spec * p.batch;
@@ -1135,7 +1187,7 @@ __global__ void __launch_bounds__(kNT) k_sweep(PipeP p, PipeBufs B, int step0, i
       ph_recon_point<T, TW>(p, B, pt, pt < n_pts);
     }
     grid.sync();
-    for (long it = blockIdx.x; it < n_planes; it += gridDim.x) ph_irecon_ifft_zy<T, TW, L, L>(p, B, it, lds);
+    for (long it = blockIdx.x; it < n_planes; it += gridDim.x) ph_irecon_ifft_zy<T, TW, L, L, kNT>(p, B, it, lds, wl);
     grid.sync();
     for (long it = blockIdx.x; it < n_tiles; it += gridDim.x) ph_ifftx_unfold<T, TW, L>(p, B, it, step, lds);
     grid.sync();
