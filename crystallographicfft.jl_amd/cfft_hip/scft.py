@@ -171,7 +171,7 @@ class SCFTSolver:
         self.chiN = float(chiN)
         path = default_path(N, ops_shifted, lattice, precision) if path is None else path
         self.plan = DevicePlan(N, ops_shifted, 1.0 / self.ns, lattice, path, precision, batch=2)
-        if axis_split:  # the per-axis chain of path QS (CFFT_OPT_AXIS_SPLIT)
+        if axis_split:  # CFFT_OPT_AXIS_SPLIT: checked by the plan, the kernels are the same
             self.plan.set_option(L.OPT_AXIS_SPLIT, 1)
         self.M = self.plan.M
         self.M3 = int(np.prod(self.M))
@@ -342,8 +342,8 @@ class SCFTEnsemble:
     """Several ``SCFTBatch`` contexts (any grids, space groups and instance
     counts; one precision and Ns; path QS with channel grids H in {8, 12, 16,
     24, 32}) advanced together through ``cfft_scft_ensemble_*``: per
-    iteration one launch per chain stage and contour step covers the plane
-    pairs (or tiles) of every context, from a work list, and the sweep is
+    iteration one launch per chain stage and contour step covers the lines
+    (or plane pairs, tiles) of every context of a kind, from a work list, and the sweep is
     replayed from one captured hipGraph.  Per instance the results are those
     of its own context bit for bit.  The batches must outlive the ensemble."""
 

@@ -9,8 +9,8 @@ schedule computes each field with the same arithmetic), only the
 decomposition of the phase kernels and how the step sequence is launched.
 The lane split R1 x R2 of a length-H transform (in-lane R2-point passes,
 then a cross-lane radix-R1 pass) reorders the butterflies, so results move
-by rounding only; it is searched only when `lanes` is set.  So does the
-per-axis chain of path QS (CFFT_OPT_AXIS_SPLIT), searched when `axis` is set.  A timing is one
+by rounding only; it is searched only when `lanes` is set.  CFFT_OPT_AXIS_SPLIT,
+searched when `axis` is set, no longer changes the kernels of a plan.  A timing is one
 contour sweep of `steps` Strang steps over `batch` fields with all
 interaction factors 1 (a plain multi-step sweep, the kernels of the stored
 sweeps apart from the q store), after one untimed sweep that captures the
@@ -38,8 +38,8 @@ def schedule_candidates(H1):
 
 def extra_dimensions(plan, lanes, axis=False):
     """Further schedule dimensions of a plan on path QS: with `axis`, the
-    per-axis chain (H = 8, 12, 16, 24, 32; plans without the separable
-    multiply refuse it and keep the plane pairs); the plane-pair workgroup size (512 threads
+    per-axis option (H = 8, 12, 16, 24, 32; plans without the separable
+    multiply refuse it); the plane-pair workgroup size (512 threads
     for H = 16, 24, 32) and, with `lanes`, the lane split R1 = 2 of the
     transforms (H = 16, 32)."""
     out = []

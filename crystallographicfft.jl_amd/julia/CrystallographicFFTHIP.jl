@@ -113,8 +113,8 @@ function DevicePlan(N::NTuple{3,Int}, ops_shifted, ds::Float64, lattice::Abstrac
     return p
 end
 
-# Launch schedule of a plan (e.g. set_option!(dev, OPT_AXIS_SPLIT, 1): the per-axis chain
-# of path QS); results do not depend on it beyond rounding.
+# Launch schedule of a plan (e.g. set_option!(dev, OPT_AXIS_SPLIT, 1), accepted as before but
+# without effect on path QS today); results do not depend on it beyond rounding.
 set_option!(dev::DevicePlan, key::Integer, value::Integer) =
     check(ccall((:cfft_plan_set_option, libcfft), Cint, (Ptr{Cvoid}, Int32, Int64),
                 dev.handle, Int32(key), Int64(value)))
