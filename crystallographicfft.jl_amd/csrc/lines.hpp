@@ -97,7 +97,10 @@ __device__ __forceinline__ void load_matrix(const double* __restrict__ m, int la
 // CU; the matrix operand's own pattern, 16 rows of 64 bytes per load, takes
 // 17, and loads straight into LDS issue at one per 120 cycles), and written
 // with chunk c of row r at chunk (c + s(r)) mod the row's chunks, s(r) chosen
-// so that the 16 rows an operand read touches lie on different banks.
+// so that the 16 rows an operand read touches lie on different banks.  The
+// chunks pass between the lanes of one wave: no workgroup barrier, but a
+// wave_sync() between the writes and the reads, and before the second round's
+// writes over rows that other lanes have read.
 template <typename T, int H>
 struct LineStage {
   static constexpr int E = 16 / (int)sizeof(T);        // values per chunk
@@ -371,6 +374,7 @@ __device__ __forceinline__ void ph_lines(const LineP& p, const double* Eo, const
 
   if constexpr (IN) {
     stage_rows<T, H>(rows, lane, own);
+    wave_sync();
     mfma_d4 a1[NT], a2[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -382,7 +386,9 @@ __device__ __forceinline__ void ph_lines(const LineP& p, const double* Eo, const
     for (int i = 0; i < KS; ++i) {
       if (i > 0 && 4 * i % S::W == 0) {  // the next round's columns, over the ones just read
         load_rows<T, H>(src + 4 * i, rs, lane, rows);
+        wave_sync();
         stage_rows<T, H>(rows, lane, own);
+        wave_sync();
       }
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
