@@ -1511,8 +1511,10 @@ EnsPlanInfo ens_plan_info(cfft_plan* p) {
 }
 
 // The same launch parameters and buffers as the plan's own history sweep
-// (cfft_sweep_hist_dev), so an ensemble computes what the plan computes.
-void ens_slot_params(cfft_plan* p, const EnsPart& part, EnsSlot* out) {
+// (cfft_sweep_hist_dev), so an ensemble computes what the plan computes.  The
+// chain is the one recorded in `made` when the ensemble took the plan: its
+// kernels are launched whatever options the plan has been given since.
+void ens_slot_params(cfft_plan* p, const EnsPlanInfo& made, const EnsPart& part, EnsSlot* out) {
   check_plan(p);
   require((int)part.E1.size() == p->batch && (int)part.E2.size() == p->batch && (int)part.sw.size() == p->batch,
           CFFT_ERR_INVALID, "one pair of interaction factors and one switch step per field");
@@ -1524,7 +1526,8 @@ void ens_slot_params(cfft_plan* p, const EnsPart& part, EnsSlot* out) {
   std::memset(static_cast<void*>(out), 0, sizeof(EnsSlot));
   out->p = pipe_params(p, es);
   out->B = pipe_bufs(p, nullptr, nullptr, p->d_F.p, false);
-  if (use_lines(p)) {
+  if (made.lines) {
+    require(p->lines_ok != 0, CFFT_ERR_INVALID, "the plan no longer has the matrices its ensemble runs on");
     out->l = line_params(p, out->p, out->B, 0, 0);
     out->le = line_ents(p, out->p);
   }

@@ -303,7 +303,7 @@ void ens_sweep_run(EnsSweep* e, const std::vector<EnsPart>& parts, const std::ve
   hip_check(hipEventSynchronize(e->staged), "hipEventSynchronize");
   for (int k = 0; k < e->n; ++k) {
     require(parts[k].plan != nullptr, CFFT_ERR_INVALID, "null plan");
-    ens_slot_params(parts[k].plan, parts[k], e->slots_h + k);
+    ens_slot_params(parts[k].plan, e->info[k], parts[k], e->slots_h + k);
   }
   // the work lists: every item of every active field (items are field-major:
   // field b of a plan owns items b * per_field .. (b + 1) * per_field - 1)

@@ -70,7 +70,8 @@ struct EnsPlanInfo {
   long M3;
 };
 EnsPlanInfo ens_plan_info(cfft_plan* p);
-void ens_slot_params(cfft_plan* p, const EnsPart& part, EnsSlot* out);
+// `made`: what ens_plan_info said when the ensemble was created.
+void ens_slot_params(cfft_plan* p, const EnsPlanInfo& made, const EnsPart& part, EnsSlot* out);
 
 struct EnsSweep;
 // Checks the parts (path QS, FP64 twiddle arithmetic, one precision, cubic

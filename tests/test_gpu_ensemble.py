@@ -63,6 +63,33 @@ def test_ensemble_iterations_equal_own_contexts(prec):
                 assert np.array_equal(x, y)
 
 
+@pytest.mark.parametrize("prec", [cf.FP64, cf.MIXED])
+@pytest.mark.parametrize("opt,value", [(cf._lib.OPT_FFT_LANES, 2)])
+def test_ensemble_keeps_its_kernels_when_options_change(prec, opt, value):
+    """A schedule option given to a member plan after the ensemble was created
+    selects other kernels for the plan's own sweeps, not for the ensemble's:
+    its iterations stay those of an untouched ensemble bit for bit (Im-3m 64^3,
+    line matrices; Fddd 64^3, plane pairs; the option set before the first and
+    between two iterations)."""
+    from cfft_hip.scft import SCFTEnsemble
+    contexts = [(229, (64, 64, 64), 4.0, [(0.30, 16.0, 21), (0.42, 22.0, 22)]), _CONTEXTS[3]]
+    made = _setup(prec, ns=20, contexts=contexts)
+    print(f"ensemble option {opt} -> {value} after creation, prec={prec}", flush=True)
+    a = SCFTEnsemble([x for x, _, _ in made])
+    b = SCFTEnsemble([y for _, y, _ in made])
+    for x, y, starts in made:
+        _set(x, starts)
+        _set(y, starts)
+    for v in (value, 0, value):
+        for x, _, _ in made:
+            x.set_schedule({opt: v})
+        assert a.iterate() == b.iterate(), v
+    for x, y, _ in made:
+        for i in range(x.n):
+            for u, v in zip(x.fields(i) + x.densities(i), y.fields(i) + y.densities(i)):
+                assert np.array_equal(u, v)
+
+
 def test_ensemble_solve_stops_each_instance():
     """solve() through the ensemble: every instance stops at its own
     convergence with the iteration count and results of its own context's
