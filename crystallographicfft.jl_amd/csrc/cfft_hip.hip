@@ -704,6 +704,13 @@ struct ESel {
   const int32_t* sw = nullptr;
 };
 
+// y rows per tile of the fold / unfold kernels: a power of two (shift/mask
+// tile indexing).
+void set_tile_rows(PipeP& pp, int yb) {
+  pp.YB = yb;
+  pp.ybs = yb == 8 ? 3 : (yb == 4 ? 2 : (yb == 2 ? 1 : 0));
+}
+
 PipeP pipe_params(cfft_plan* p, const ESel& es) {
   PipeP pp;
   std::memset(&pp, 0, sizeof(pp));  // padding too: the bytes key the graph cache
@@ -720,12 +727,10 @@ PipeP pipe_params(cfft_plan* p, const ESel& es) {
     pp.chbits |= (uint32_t)(p->chmap[i] >= 0 ? p->chmap[i] : 15) << (4 * i);
   }
   pp.batch = p->batch;
-  // y rows per tile: a power of two (shift/mask tile indexing), by default the
-  // largest <= 8 dividing H1; n_ch * YB <= 64 rows fit the tile's LDS
+  // by default the largest <= 8 dividing H1; n_ch * YB <= 64 rows fit the tile's LDS
   int yb = p->tile_rows ? p->tile_rows : 8;
   while (p->H[1] % yb) yb >>= 1;
-  pp.YB = yb;
-  pp.ybs = yb == 8 ? 3 : (yb == 4 ? 2 : (yb == 2 ? 1 : 0));
+  set_tile_rows(pp, yb);
   pp.n_spec = p->n_spec;
   pp.d = p->d;
   pp.P = p->P;
@@ -1504,7 +1509,9 @@ EnsPlanInfo ens_plan_info(cfft_plan* p) {
   i.lanes = p->lanes;
   i.axis_split = p->axis_split;
   i.pair_items = (long)p->qs_items * p->batch;
-  i.tile_items = n_tiles(p, pipe_params(p, ESel{}));
+  const PipeP pp = pipe_params(p, ESel{});
+  i.tile_rows = pp.YB;
+  i.tile_items = n_tiles(p, pp);
   i.line_items = (long)p->batch * p->H[0] * line_parts(p->H[0]);
   i.M3 = p->M3;
   return i;
@@ -1512,8 +1519,9 @@ EnsPlanInfo ens_plan_info(cfft_plan* p) {
 
 // The same launch parameters and buffers as the plan's own history sweep
 // (cfft_sweep_hist_dev), so an ensemble computes what the plan computes.  The
-// chain is the one recorded in `made` when the ensemble took the plan: its
-// kernels are launched whatever options the plan has been given since.
+// chain and the tile height are those recorded in `made` when the ensemble
+// took the plan: its kernels and work lists were laid out for them, whatever
+// options the plan has been given since.
 void ens_slot_params(cfft_plan* p, const EnsPlanInfo& made, const EnsPart& part, EnsSlot* out) {
   check_plan(p);
   require((int)part.E1.size() == p->batch && (int)part.E2.size() == p->batch && (int)part.sw.size() == p->batch,
@@ -1525,6 +1533,7 @@ void ens_slot_params(cfft_plan* p, const EnsPlanInfo& made, const EnsPart& part,
   es.sw = part.sw.data();
   std::memset(static_cast<void*>(out), 0, sizeof(EnsSlot));
   out->p = pipe_params(p, es);
+  set_tile_rows(out->p, made.tile_rows);
   out->B = pipe_bufs(p, nullptr, nullptr, p->d_F.p, false);
   if (made.lines) {
     require(p->lines_ok != 0, CFFT_ERR_INVALID, "the plan no longer has the matrices its ensemble runs on");

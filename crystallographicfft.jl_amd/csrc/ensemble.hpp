@@ -65,6 +65,7 @@ struct EnsPlanInfo {
   int lines;                    // line-matrix chain: 1 + centring; 0: the plane-pair chain
   int lanes;                    // path QS: a lane split other than the default (0: none)
   int axis_split;               // CFFT_OPT_AXIS_SPLIT is set (ensembles refuse such plans)
+  int tile_rows;                // y rows per fold / unfold tile
   long pair_items, tile_items;  // plane-pair and tile work items of one launch
   long line_items;              // work items of one launch of the line-matrix chain
   long M3;

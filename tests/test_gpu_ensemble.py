@@ -64,11 +64,11 @@ def test_ensemble_iterations_equal_own_contexts(prec):
 
 
 @pytest.mark.parametrize("prec", [cf.FP64, cf.MIXED])
-@pytest.mark.parametrize("opt,value", [(cf._lib.OPT_FFT_LANES, 2)])
+@pytest.mark.parametrize("opt,value", [(cf._lib.OPT_FFT_LANES, 2), (cf._lib.OPT_TILE_ROWS, 2)])
 def test_ensemble_keeps_its_kernels_when_options_change(prec, opt, value):
     """A schedule option given to a member plan after the ensemble was created
-    selects other kernels for the plan's own sweeps, not for the ensemble's:
-    its iterations stay those of an untouched ensemble bit for bit (Im-3m 64^3,
+    selects other kernels or tiles for the plan's own sweeps, not for the
+    ensemble's, whose work lists were laid out before: its iterations stay those of an untouched ensemble bit for bit (Im-3m 64^3,
     line matrices; Fddd 64^3, plane pairs; the option set before the first and
     between two iterations)."""
     from cfft_hip.scft import SCFTEnsemble
