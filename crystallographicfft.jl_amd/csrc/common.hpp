@@ -27,8 +27,12 @@ std::recursive_mutex& setup_mutex();
 
 
 inline void hip_check(hipError_t e, const char* what) {
-  if (e != hipSuccess)
+  if (e != hipSuccess) {
+    // reported here: the runtime keeps it as the thread's last error, which the
+    // check after a later launch would take for its own
+    (void)hipGetLastError();
     throw Error{CFFT_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e)};
+  }
 }
 
 template <typename F>

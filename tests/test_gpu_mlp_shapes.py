@@ -61,3 +61,20 @@ def test_layers(dims, rows):
     for n in [a * b for a, b in zip(dims[:-1], dims[1:])] + dims[1:]:
         assert np.linalg.norm(g[off:off + n] - gr[off:off + n]) <= 2.0 ** -6 * np.linalg.norm(gr[off:off + n])
         off += n
+
+
+def test_refused_allocation_is_reported_once():
+    """A batch whose activations cannot be allocated (15 TB) is refused on the
+    host; the next launches, of another object, do not report it again."""
+    import cfft_hip as cf
+    net, _ = _net([6, 512, 512, 512, 256], 13)
+    x, t = np.ones((8, 6), np.float32), np.ones((8, 256), np.float32)
+    N = (32, 32, 32)
+    _, ops_s = cf.find_optimal_shift(cf.get_ops(229, 3, N), N)
+    plan = cf.DevicePlan(N, ops_s, 0.01, 4.0 * np.eye(3), cf.PATH_M7, cf.FP64)
+    f = np.random.default_rng(3).standard_normal(plan.M)
+    want = plan.diffuse(f)
+    with pytest.raises(cf.CFFTError) as e:
+        net.train(x, t, epochs=1, batch=2 ** 31 - 1)
+    assert e.value.code == cf._lib.CFFT_ERR_HIP
+    assert np.array_equal(plan.diffuse(f), want)
