@@ -375,7 +375,7 @@ namespace {
 
 void ensure_rows(cfft_mlp* p, int rows) {
   if (rows <= p->max_rows) return;
-  p->max_rows = rows;
+  p->max_rows = 0;  // until every buffer is there: a failed allocation leaves some without memory
   long tot = 0;
   p->zoff.assign(p->L + 1, 0);
   for (int l = 0; l < p->L; ++l) {
@@ -391,6 +391,7 @@ void ensure_rows(cfft_mlp* p, int rows) {
   p->dB.alloc(4L * rows * dmax);
   p->xt.alloc(4L * rows * (p->dims[0] + p->dims[p->L]));
   p->part.alloc(8L * tiles(rows, 16) * tiles(p->dims[p->L], 16));
+  p->max_rows = rows;
 }
 
 float* Zl(cfft_mlp* p, int l) { return static_cast<float*>(p->Z.p) + p->zoff[l]; }

@@ -78,3 +78,20 @@ def test_refused_allocation_is_reported_once():
         net.train(x, t, epochs=1, batch=2 ** 31 - 1)
     assert e.value.code == cf._lib.CFFT_ERR_HIP
     assert np.array_equal(plan.diffuse(f), want)
+
+
+def test_failed_allocation_leaves_the_network_usable():
+    """A batch whose activations cannot be allocated (15 TB) is refused on the
+    host; the calls after it allocate their own and compute as before."""
+    import cfft_hip as cf
+    dims = [6, 512, 512, 512, 256]
+    net, _ = _net(dims, 13)
+    rng = np.random.default_rng(13)
+    x = rng.standard_normal((8, 6)).astype(np.float32)
+    t = rng.standard_normal((8, 256)).astype(np.float32)
+    loss, g = net.gradient(x, t)
+    with pytest.raises(cf.CFFTError) as e:
+        net.train(x, t, epochs=1, batch=2 ** 31 - 1)
+    assert e.value.code == cf._lib.CFFT_ERR_HIP
+    loss2, g2 = net.gradient(x, t)
+    assert loss2 == loss and np.array_equal(g2, g)
