@@ -115,12 +115,14 @@ __device__ __forceinline__ void lds_fft(cx<T>* buf, int n_tr, int ts, int es) {
 // `step`: FP64 in both precisions (an FP32 rounding of E would be the same
 // relative error at a point on every step, compounding along the contour
 // instead of averaging out).  Every candidate is read before the choice
-// (selects, no branches), so the reads issue together.
+// (selects, no branches), so the reads issue together; a contiguous array may
+// serve more entries than the tables of pointers hold.
 __device__ __forceinline__ const double* pipe_E(const PipeP& p, int b, int step, long M3) {
   const void* c0 = p.E1[0];
-  const void* e1 = p.E1[b];
-  const void* e2 = p.E2[b];
-  const int sw = p.sw[b];
+  const int k = b < kMaxEPtr ? b : 0;
+  const void* e1 = p.E1[k];
+  const void* e2 = p.E2[k];
+  const int sw = p.sw[k];
   const double* contig = c0 ? static_cast<const double*>(c0) + b * M3 : nullptr;
   const double* split = static_cast<const double*>(step < sw ? e1 : e2);
   return p.E_contig ? contig : split;

@@ -207,6 +207,23 @@ def test_step_and_batch(sg):
         assert rel(outb[b], single) < 1e-15
 
 
+@pytest.mark.parametrize("path", [cf.PATH_M7, cf.PATH_QS])
+def test_more_fields_than_factor_pointers(path):
+    """A batch of 70 fields (the tables of per-field factor pointers hold 64):
+    its steps, with one contiguous array of factors, equal those of the same
+    fields in batches of 35 bit for bit."""
+    N = (32, 32, 32)
+    _, ops_s = cf.find_optimal_shift(cf.get_ops(229, 3, N), N)
+    many = cf.DevicePlan(N, ops_s, DS, LAT4, path, batch=70)
+    half = cf.DevicePlan(N, ops_s, DS, LAT4, path, batch=35)
+    rng = np.random.default_rng(70)
+    q, w = rng.standard_normal((70,) + many.M), rng.standard_normal((70,) + many.M)
+    for nsteps in (1, 3):
+        got = many.step(q, w, DS, nsteps=nsteps)
+        want = np.concatenate([half.step(q[:35], w[:35], DS, nsteps=nsteps), half.step(q[35:], w[35:], DS, nsteps=nsteps)])
+        assert np.array_equal(got, want)
+
+
 @pytest.mark.parametrize("sg", [229, 230, 47, 70])
 def test_mixed_precision(sg):
     N = (32, 32, 32)
