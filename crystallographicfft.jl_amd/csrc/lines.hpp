@@ -206,6 +206,13 @@ struct LineLds {
   static constexpr int CH = PTS > ST ? PTS : ST, BYTES = LineCent<CENT>::NCH * CH;
 };
 
+// VX neighbouring values of a caller's array, which is aligned to its element
+// only (the plan's own channels are aligned to whole vectors).
+template <typename T, int VX>
+struct CallerVec {
+  typedef T type __attribute__((ext_vector_type(VX), aligned(sizeof(T))));
+};
+
 template <int N>
 __device__ __forceinline__ void wht(double (&v)[N]) {
 #pragma unroll
@@ -231,7 +238,7 @@ __device__ __forceinline__ void line_point(double (&g)[LineCent<CENT>::NCH][VX],
 #pragma clang fp contract(off)
   constexpr int NCH = LineCent<CENT>::NCH;
   constexpr unsigned M = 2 * H;
-  typedef T vec __attribute__((ext_vector_type(VX)));
+  typedef typename CallerVec<T, VX>::type vec;
   double u[VX][NCH], h[VX][NCH];
   bool seen[NCH] = {};
 #pragma unroll
@@ -281,7 +288,7 @@ __device__ __forceinline__ void line_point(double (&g)[LineCent<CENT>::NCH][VX],
 template <typename T, int H, int VX>
 __device__ __forceinline__ void load_corner(const T* __restrict__ f, unsigned at, int e, double (&v)[VX]) {
   constexpr unsigned M = 2 * H;
-  typedef T vec __attribute__((ext_vector_type(VX)));
+  typedef typename CallerVec<T, VX>::type vec;
   const unsigned corner = (unsigned)(((e & 1) + ((e >> 1) & 1) * M + (e >> 2) * M * M) * H);
   const vec t = *reinterpret_cast<const vec*>(f + at + corner);
 #pragma unroll

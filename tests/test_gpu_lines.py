@@ -87,3 +87,29 @@ def test_update_kernel_reaches_matrices():
     plan.update_kernel(0.02, lat)
     fresh = cf.DevicePlan(N, ops_s, 0.02, lat, cf.PATH_QS, cf.FP64)
     assert np.array_equal(plan.step(q, w, 0.02, nsteps=3), fresh.step(q, w, 0.02, nsteps=3))
+
+
+@pytest.mark.parametrize("n", [64, 128])
+@pytest.mark.parametrize("prec", [cf.FP64, cf.MIXED])
+def test_element_aligned_pointers(n, prec):
+    """Field and factor pointers are aligned to one element only: arrays that
+    start one element past a vector's boundary give the bits of arrays that
+    start on it (Im-3m: one point per thread at 64^3, two at 128^3)."""
+    import torch
+    N = (n, n, n)
+    _, ops_s = cf.find_optimal_shift(cf.get_ops(229, 3, N), N)
+    plan = cf.DevicePlan(N, ops_s, DS, 4.0 * np.eye(3), cf.PATH_QS, prec)
+    m = int(np.prod(plan.M))
+    dt = torch.float64 if prec == cf.FP64 else torch.float32
+    rng = np.random.default_rng(n)
+    q, E = torch.from_numpy(rng.standard_normal(m)), torch.from_numpy(rng.uniform(0.5, 1.5, m))
+    got = []
+    for off in (0, 1):
+        qd, Ed = torch.zeros(m + 2, dtype=dt, device="cuda"), torch.zeros(m + 2, dtype=torch.float64, device="cuda")
+        qd[off:off + m] = q.to("cuda", dt)
+        Ed[off:off + m] = E.to("cuda")
+        plan.step_dev(qd[off:].data_ptr(), Ed[off:].data_ptr(), 3, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert qd[:off].abs().sum() == 0 and qd[off + m:].abs().sum() == 0
+        got.append(qd[off:off + m].cpu())
+    assert torch.equal(got[0], got[1])
