@@ -35,7 +35,7 @@ __device__ __forceinline__ const EnsSlot& ens_slot(const EnsSlot* S, int k) {
 // all batch entries) * parts + part), as launched by the plan's own sweep:
 // kLinesOut alone folds slice 0, otherwise q(step + 1) goes to its slice.
 template <typename T, int L, int CENT, int MODE>
-__global__ void __launch_bounds__(64 * LineCent<CENT>::NCH, line_waves(L))
+__global__ void __launch_bounds__(64 * LineCent<CENT>::NCH, line_waves(L, LineCent<CENT>::NCH))
     k_lines_ens(const EnsSlot* __restrict__ S, const int* __restrict__ count, const EnsWork* __restrict__ work,
                 int step, int flags) {
   constexpr int NPART = line_parts(L);

@@ -353,8 +353,14 @@ __device__ __forceinline__ void ph_lines(const LineP& p, const double* Eo, const
   }
   const bool other_E = IN && OUT && En != Eo;
   const double* tl = p.mats + (line * 4 + ((av >> (2 * line)) & 3)) * VAR;
+  // eight waves of a workgroup leave 256 registers each, and 128 of line matrix
+  // beside the staged FP64 rows spilled up to 37: read where a pass takes it, not
+  // held across the others (Pm-3m 256^3, 1 and 2 fields 29.3, 54.8 -> 24.3, 44.2 us)
+  constexpr bool LATE = NT * KS >= 64 && NCH == 8 && sizeof(T) == 8;
+  if constexpr (!LATE) {
 #pragma unroll
-  for (int t = 0; t < NT; ++t) load_matrix<KS>(tl + t * (KS * 64), lane, ml[t]);
+    for (int t = 0; t < NT; ++t) load_matrix<KS>(tl + t * (KS * 64), lane, ml[t]);
+  }
   // en: the factor of the fold when it is another array (or the field, without IN)
   double eo[NPT][8][VX], en[NPT][8][VX];
   unsigned at[NPT];
@@ -403,6 +409,11 @@ __device__ __forceinline__ void ph_lines(const LineP& p, const double* Eo, const
         const double gv = staged<T, H>(own, H % 16 == 0 || row < H ? row : H - 1, 4 * i % S::W + g);
         a1[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(gv, mx[i], a1[t], 0, 0, 0);
       }
+    }
+    if constexpr (LATE) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) load_matrix<KS>(tl + t * (KS * 64), lane, ml[t]);
     }
     // the line matrix: result register j of tile t is line position
     // 16 t + 4 j + l / 16, the B operand of k-step 4 t + j
@@ -485,6 +496,11 @@ __device__ __forceinline__ void ph_lines(const LineP& p, const double* Eo, const
     }
   }
   if constexpr (OUT) {
+    if constexpr (LATE) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) load_matrix<KS>(tl + t * (KS * 64), lane, ml[t]);
+    }
     __syncthreads();
     mfma_d4 a3[NT];
 #pragma unroll
@@ -525,13 +541,17 @@ __host__ __device__ __forceinline__ void lines_item(unsigned parts, unsigned blk
 // Factors of batch entry b at `step`.
 __device__ __forceinline__ const double* line_E(const LineEnt::Entry& e, int step) { return step < e.sw ? e.e1 : e.e2; }
 
-// Three waves per SIMD where the registers allow it: below that the compiler
-// moves the accumulators through the second register file (Im-3m 128^3, 2
-// fields FP64 6.1 -> 5.8 us, 16 fields mixed 13.6 -> 11.9).
-constexpr int line_waves(int H) { return H <= 32 ? 3 : 1; }
+// Three waves per SIMD for H <= 32: below that the compiler moves the
+// accumulators through the second register file (Im-3m 128^3, 2 fields FP64
+// 6.1 -> 5.8 us, 16 fields mixed 13.6 -> 11.9).  Two with two channels, whose
+// threads hold two pairs of points at H = 24 and 32: three spilled 4 to 124
+// registers (Fm-3m 128^3, 1, 2, 8 fields FP64 6.5, 6.8, 11.5 -> 5.4, 5.6, 8.6 us,
+// mixed 5.4, 5.6, 8.8 -> 5.1, 5.2, 7.8; 96^3 5.28, 5.34, 7.4 -> 5.12, 5.19, 7.2).
+// No instance has scratch memory.
+constexpr int line_waves(int H, int nch) { return H <= 32 ? (H > 16 && nch == 2 ? 2 : 3) : 1; }
 
 template <typename T, int H, int CENT, int MODE>
-__global__ void __launch_bounds__(64 * LineCent<CENT>::NCH, line_waves(H))
+__global__ void __launch_bounds__(64 * LineCent<CENT>::NCH, line_waves(H, LineCent<CENT>::NCH))
     k_lines(void* ch, const double* mats, unsigned long long axv, int batch, int step, int flags, const double* E,
             const void* f0_in, void* f0_out, LineEnt ents) {
   __shared__ __align__(16) unsigned char lds[LineLds<T, H, CENT, MODE>::BYTES];

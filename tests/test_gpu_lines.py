@@ -25,7 +25,7 @@ def _rel(a, b):
 
 
 FP64_CASES = [(47, 32), (229, 32), (225, 32), (229, 48), (65, 48), (230, 48), (230, 64), (225, 64), (47, 96), (230, 96),
-              (229, 128), (71, 192)]
+              (229, 128), (71, 192), (225, 96), (225, 128)]
 MIXED_CASES = [(47, 32), (65, 48), (230, 64), (225, 96)]
 
 
