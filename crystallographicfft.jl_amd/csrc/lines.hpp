@@ -33,6 +33,12 @@ namespace cfft {
 
 typedef double mfma_d4 __attribute__((ext_vector_type(4)));
 
+// Channel lengths of the chain: at every one it beats the plane-pair chain, in
+// each centring, precision and batch.  Steps of one field, FP64, plane pairs ->
+// line matrices: Pmmm H = 8 10.0 -> 3.6 us, 16 11.4 -> 4.3, 32 18.2 -> 8.0, 48
+// 41.2 -> 15.7; Pm-3m H = 64 71.1 -> 24.3; Im-3m H = 48 31.6 -> 10.1, 64 52.0 ->
+// 14.7; Fm-3m H = 48 27.0 -> 8.5, 64 49.0 -> 13.0; eight fields of Pmmm, H = 32
+// 45.3 -> 15.3; two of Im-3m, H = 64 89.0 -> 26.5 (mixed 63.4 -> 23.6).
 constexpr int kLineLens[] = {8, 12, 16, 24, 32, 48, 64};
 inline bool line_len_ok(int H) {
   for (int v : kLineLens)
@@ -194,8 +200,9 @@ enum { kLinesIn = 1, kLinesOut = 2, kLinesStore = 4 };
 
 // x-values per workgroup: the matrix instructions' tile.  Measured against 8
 // (every CU at work from half the fields, half of each tile wasted) and 32
-// (a plane's rows read once): Im-3m 128^3 FP64 at 1, 2, 8, 16 fields 5.58,
-// 6.01, 12.1 us (8), 5.75, 6.11, 8.9, 15.7 us (16), 7.7, 8.1, 9.6, 14.8 us (32).
+// (a plane's rows read once): Im-3m 128^3 FP64 at 1, 2 and 8 fields 5.58, 6.01,
+// 12.1 us (8), 5.75, 6.11, 8.9 us (16), 7.7, 8.1, 9.6 us (32); at 16 fields
+// 15.7 us (16), 14.8 us (32).
 constexpr int kCW = 16;
 constexpr int line_parts(int H) { return (H + kCW - 1) / kCW; }
 
