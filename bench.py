@@ -82,11 +82,8 @@ def stage_bytes(plan, e, lines=False):
     }
 
 
-def launch_bytes(plan, e, stage, steps_per_launch, lines=False):
-    """Algorithmic bytes of one launch of `stage` (the persistent sweep moves
-    one Strang step's bytes per field per contour step)."""
-    if stage == "sweep":
-        return steps_per_launch * plan.batch * step_bytes(plan, e)
+def launch_bytes(plan, e, stage, lines=False):
+    """Algorithmic bytes of one launch of `stage`."""
     return stage_bytes(plan, e, lines)[stage]
 
 
@@ -149,7 +146,7 @@ def profile_stages(sw, steps, torch):
     return {name: (float(ms[i]), int(cnt[i])) for i, name in enumerate(L.STAGES) if cnt[i]}
 
 
-STRATEGY_PATH = {"m7_chain": 0, "m7_persistent": 0, "qr_chain": 5, "qs_chain": 6, "qs_chain_eager": 6,
+STRATEGY_PATH = {"m7_chain": 0, "qr_chain": 5, "qs_chain": 6, "qs_chain_eager": 6,
                  "qs_chain_axis": 6, "qs_chain_tuned": 6}
 # the FETCH_SIZE / WRITE_SIZE record of each pipeline path's chain kernels
 # (eager launches and graph replays run the same kernels)
@@ -680,21 +677,19 @@ def main():
     variants = {}
     for name, prec, e in (("fp64", cf.FP64, 8), ("mixed", cf.MIXED, 4)):
         # launch strategies: the centred fwd+K+bwd chain (one launch per phase,
-        # hipGraph replay) or one cooperative launch per sweep, and the
-        # orbit-reduced Q chain; the fastest one is used for the timed region
+        # hipGraph replay), the orbit-reduced Q chain and path QS; the fastest
+        # one is used for the timed region
         trial = {}
         sweeps = {}
         # the plane-pair chain's schedule (tile rows, graph replay, pair
         # workgroup size, lane split) tuned on this workload (cfft_hip.tune)
         from cfft_hip.tune import tune_schedule
         tuned, tuned_times = tune_schedule(N, ops_s, lat, NS, prec, 2, cf.PATH_QS, lanes=True, axis=True)
-        for label, path, persist, graph in (("m7_chain", cf.PATH_AUTO, 0, 1), ("m7_persistent", cf.PATH_AUTO, 1, 1),
-                                            ("qr_chain", cf.PATH_QR, 0, 1), ("qs_chain", cf.PATH_QS, 0, 1),
-                                            ("qs_chain_eager", cf.PATH_QS, 0, 0), ("qs_chain_axis", cf.PATH_QS, 0, 1),
-                                            ("qs_chain_tuned", cf.PATH_QS, 0, 1)):
+        for label, path, graph in (("m7_chain", cf.PATH_AUTO, 1), ("qr_chain", cf.PATH_QR, 1),
+                                   ("qs_chain", cf.PATH_QS, 1), ("qs_chain_eager", cf.PATH_QS, 0),
+                                   ("qs_chain_axis", cf.PATH_QS, 1), ("qs_chain_tuned", cf.PATH_QS, 1)):
             sw = cf.scft.PropagatorSweep(N, ops_s, lat, F_A, NS, prec, path=path)
             sw.set_fields(wA, wB)
-            sw.plan.set_option(cf._lib.OPT_PERSISTENT, persist)
             sw.plan.set_option(cf._lib.OPT_GRAPH, graph)
             if label == "qs_chain_axis":  # the per-axis chain of path QS
                 sw.plan.set_option(cf._lib.OPT_AXIS_SPLIT, 1)
@@ -726,10 +721,10 @@ def main():
             scratch = sw.q.clone()
             avg_ms = live_launch_ms(sw.plan, dom, scratch.data_ptr(), sw._E1, sw.stream())
             del scratch
-        else:  # persistent sweep: one event pair around each cooperative launch
+        else:
             avg_ms = stages[dom][0] / stages[dom][1]
         lines = line_chain(stages)
-        nb = launch_bytes(sw.plan, e, dom, NS, lines)
+        nb = launch_bytes(sw.plan, e, dom, lines)
         achieved = nb / (avg_ms * 1e-3) / 1e9
         # every per-step chain kernel beside the dominant one, timed the same way
         chain = {}
@@ -739,7 +734,7 @@ def main():
             scratch = sw.q.clone()
             ms = avg_ms if st == dom else live_launch_ms(sw.plan, st, scratch.data_ptr(), sw._E1, sw.stream())
             del scratch
-            b = launch_bytes(sw.plan, e, st, NS, lines)
+            b = launch_bytes(sw.plan, e, st, lines)
             chain[st] = {"avg_launch_ms": ms, "bytes_per_launch": b, "achieved": b / (ms * 1e-3) / 1e9,
                          "frac": b / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS}
         res[name] = dict(el=el, med=med, Qq=Qq, Qd=Qd, q=qfields, stages=stages, dom=dom, avg_ms=avg_ms,

@@ -62,7 +62,6 @@ struct cfft_plan {
   int n_sym = 0;
   std::vector<int32_t> fmap_host;
   // options (cfft_plan_set_option)
-  int persistent = 0;  // contour sweeps as one cooperative launch
   int fuse = 1;        // fuse P5 of a step with P1 of the next
   int graph = 1;       // replay multi-step chains from captured hipGraphs
   int tile_rows = 0;   // y rows per fold/unfold tile (0: the default rule)
@@ -1151,41 +1150,6 @@ void run_diffuse(cfft_plan* p, const T* in, T* out_f0, const PipeP& pp, int step
   run_backward<T>(p, pp, F, out_f0, step, s, w.ch);
 }
 
-// Persistent cooperative sweep of nsteps Strang steps (cubic H-grids, fwd+K+bwd
-// paths); returns false when it cannot be used so the caller falls back to
-// one launch per phase.
-template <typename T>
-bool run_sweep_persistent(cfft_plan* p, T* q, const PipeP& pp, int step0, int nsteps, hipStream_t s) {
-  if (!p->persistent || !cubic(p) || is_q_path(p)) return false;
-  const void* kern = nullptr;
-#define CFFT_SW(L) \
-  case L: kern = reinterpret_cast<const void*>(&k_sweep<T, double, L>); break;
-  switch (p->H[0]) {
-    CFFT_SW(2) CFFT_SW(3) CFFT_SW(4) CFFT_SW(6) CFFT_SW(8) CFFT_SW(12) CFFT_SW(16) CFFT_SW(24)
-    CFFT_SW(32) CFFT_SW(48) CFFT_SW(64)
-    default: return false;
-  }
-#undef CFFT_SW
-  int dev = 0, ncu = 0, per_cu = 0, coop = 0;
-  hip_check(hipGetDevice(&dev), "hipGetDevice");
-  hip_check(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev), "attr");
-  if (!coop) return false;
-  hip_check(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "attr");
-  hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kNT, 0), "occupancy");
-  if (per_cu < 1) return false;
-  long want = std::max(n_tiles(p, pp), n_planes(p));
-  want = std::max(want, (8L * p->n_spec * p->batch + kNT - 1) / kNT);
-  const long grid = std::min<long>((long)per_cu * ncu, want);
-  PipeBufs B = pipe_bufs(p, q, q, p->d_F.p, true);
-  PipeP ppc = pp;
-  int s0 = step0, ns = nsteps;
-  void* args[] = {&ppc, &B, &s0, &ns};
-  StageTimer st(p, s, CFFT_STAGE_SWEEP);
-  hip_check(hipLaunchCooperativeKernel(kern, dim3((unsigned)grid), dim3(kNT), args, 0, s),
-            "hipLaunchCooperativeKernel");
-  return true;
-}
-
 // Projection of subgrid fields onto those invariant under the ops that keep
 // the subgrid (ops: n_sym x 12 int32, R' row-major then t'; the identity is
 // one of them): out(x) = mean_g in(R' x + t' mod M).  Fields of M0 M1 M2
@@ -1414,7 +1378,6 @@ template <typename T>
 void run_steps(cfft_plan* p, T* q, const ESel& es, int step0, int nsteps, hipStream_t s) {
   PipeP pp = pipe_params(p, es);
   if (nsteps <= 0) return;
-  if (run_sweep_persistent<T>(p, q, pp, step0, nsteps, s)) return;
   dispatch_steps<T>(p, q, 0, pp, step0, nsteps, s);
 }
 
@@ -2034,7 +1997,7 @@ int cfft_plan_set_option(cfft_plan* p, int32_t key, int64_t value) {
   return guarded([&] {
     check_plan(p);
     switch (key) {
-      case CFFT_OPT_PERSISTENT: p->persistent = value != 0; break;
+      case CFFT_OPT_PERSISTENT: break;  // accepted; sweeps are launch chains
       case CFFT_OPT_FUSE: p->fuse = value != 0; break;
       case CFFT_OPT_GRAPH: p->graph = value != 0; break;
       case CFFT_OPT_TILE_ROWS:

@@ -10,12 +10,10 @@
 //   P4  inverse recon + IFFT z, IFFT y   plane (b, c, x)   F -> ch
 //   P5  IFFT x + unfold + E      tile (b, z, y-block)      ch -> f0
 //
-// Each phase is a device function over one work item, used both by one
-// kernel per phase and by the persistent sweep kernel (grid-wide barriers
-// between phases).
+// Each phase is a device function over one work item, launched by one kernel
+// per phase and by the multi-plan kernels of the ensembles.
 #pragma once
 
-#include <hip/hip_cooperative_groups.h>
 #include <hip/hip_runtime.h>
 
 #include "fft.hpp"
@@ -1160,40 +1158,6 @@ __global__ void __launch_bounds__(kNT) k_p51(PipeP p, PipeBufs B, int step) {
   __shared__ cx<T> lds[64 * kRow<T, L0>];
   const long item = p51_item(blockIdx.x, gridDim.x, p.H[1] / p.YB, p.YB * (int)sizeof(cx<T>) < 128);
   ph_unfold_fold<T, TW, L0, STORE, LANES>(p, B, item, step, lds);
-}
-
-// ---- persistent sweep: nsteps Strang steps in one cooperative launch ---------
-// f0 is advanced in place (P1 reads it, P5 overwrites it after the barrier
-// that follows P4).  Work items are distributed grid-stride over the resident
-// workgroups; every workgroup reaches every barrier.
-template <typename T, typename TW, int L>
-__global__ void __launch_bounds__(kNT) k_sweep(PipeP p, PipeBufs B, int step0, int nsteps) {
-  namespace cg = cooperative_groups;
-  cg::grid_group grid = cg::this_grid();
-  constexpr int TILE = 64 * (L + 1);
-  constexpr int PLANE = L * (L + 1);
-  __shared__ cx<T> lds[TILE > PLANE ? TILE : PLANE];
-  __shared__ cx<TW> wl[kPhases];
-  const long n_tiles = (long)p.batch * p.H[2] * (p.H[1] / p.YB);
-  const long n_planes = (long)p.batch * p.n_ch * p.H[0];
-  const long n_pts = (long)p.n_spec * p.batch;
-  const long n_oct = (n_pts * 8 + kNT - 1) / kNT;  // workgroup-chunks of P3
-  for (int s = 0; s < nsteps; ++s) {
-    const int step = step0 + s;
-    for (long it = blockIdx.x; it < n_tiles; it += gridDim.x) ph_fold_fftx<T, TW, L>(p, B, it, step, lds);
-    grid.sync();
-    for (long it = blockIdx.x; it < n_planes; it += gridDim.x) ph_fft_yz<T, TW, L, L>(p, B, it, lds);
-    grid.sync();
-    for (long it = blockIdx.x; it < n_oct; it += gridDim.x) {
-      const long pt = (it * kNT + threadIdx.x) >> 3;
-      ph_recon_point<T, TW>(p, B, pt, pt < n_pts);
-    }
-    grid.sync();
-    for (long it = blockIdx.x; it < n_planes; it += gridDim.x) ph_irecon_ifft_zy<T, TW, L, L, kNT>(p, B, it, lds, wl);
-    grid.sync();
-    for (long it = blockIdx.x; it < n_tiles; it += gridDim.x) ph_ifftx_unfold<T, TW, L>(p, B, it, step, lds);
-    grid.sync();
-  }
 }
 
 }  // namespace cfft

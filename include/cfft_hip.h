@@ -205,9 +205,7 @@ int cfft_step_ptrs_dev(cfft_plan* plan, void* q, const void* const* E, int32_t n
 /* Contour sweep: nsteps Strang steps q <- E D (E q), batch entry b using
  * E1[b] at absolute step indices < sw[b] and E2[b] after (host arrays of
  * `batch` device pointers / ints, batch <= 64; steps are numbered from step0).
- * No counterpart in the reference (it has no SCFT driver); on cubic H-grids
- * the whole sweep is one cooperative launch with grid barriers between the
- * pipeline phases. */
+ * No counterpart in the reference (it has no SCFT driver). */
 int cfft_sweep_dev(cfft_plan* plan, void* q, const void* const* E1, const void* const* E2,
                    const int32_t* sw, int32_t step0, int32_t nsteps, void* stream);
 /* Projection of n_fields FP64 subgrid fields (M^3 each, x fastest, one after
@@ -233,7 +231,7 @@ int cfft_exp_dev(cfft_plan* plan, const void* w, void* E, double factor, int64_t
 #define CFFT_STAGE_IFFT_Z 8 /* z pass (non-cubic) / Q-path IFFT z,y  */
 #define CFFT_STAGE_UNFOLD 9 /* P5: IFFT x + unfold + E               */
 #define CFFT_STAGE_QMUL 10
-#define CFFT_STAGE_SWEEP 11 /* persistent sweep (all phases, all steps) */
+#define CFFT_STAGE_SWEEP 11 /* (unused)                              */
 #define CFFT_STAGE_UNFOLD_FOLD 12 /* P5 of step s fused with P1 of s + 1 */
 #define CFFT_STAGE_PLANE_Q 13     /* path QS: FFT y, z + Q + IFFT z, y      */
 #define CFFT_N_STAGES 14
@@ -263,9 +261,9 @@ int cfft_sweep_hist_dev(cfft_plan* plan, void* hist, const void* const* E1, cons
                         const int32_t* sw, int32_t step0, int32_t nsteps, void* stream);
 
 /* ---- plan options -------------------------------------------------------- */
-/* value != 0: run cfft_sweep_dev / cfft_step_dev on cubic H-grids as one
- * cooperative launch with grid barriers between phases (default 0: one
- * launch per phase and step). */
+/* Accepted and without effect: sweeps and multi-step calls run as chains of
+ * launches (CFFT_OPT_GRAPH replays them).  It selected one cooperative launch
+ * with grid barriers between the phases, slower at every size. */
 #define CFFT_OPT_PERSISTENT 1
 /* value != 0 (default 1): in multi-step calls, fuse the unfold of a step with
  * the fold of the next (one tile kernel, q(s + 1) is not read back). */

@@ -1,5 +1,5 @@
-"""GPU contour sweeps (cfft_sweep_dev, persistent cooperative kernel on cubic
-grids, one launch per phase otherwise) vs the oracle's Strang propagation."""
+"""GPU contour sweeps (cfft_sweep_dev, chains of launches; CFFT_OPT_PERSISTENT is
+accepted without effect) vs the oracle's Strang propagation."""
 import numpy as np
 import pytest
 
