@@ -831,6 +831,18 @@ void launch_p3(cfft_plan* p, const PipeP& pp, const PipeBufs& B, hipStream_t s) 
   launch_check<T>("k_p3");
 }
 
+template <typename T, int L>
+void launch_p4_len(const PipeP& pp, const PipeBufs& B, unsigned g, bool many, hipStream_t s) {
+  constexpr int NT = p4_threads(L * L, sizeof(T)), NTM = p4_threads(L * L, sizeof(T), true);
+  if constexpr (NTM != NT) {
+    if (many) {
+      hipLaunchKernelGGL((k_p4<T, double, L, L, NTM>), dim3(g), dim3(NTM), 0, s, pp, B);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_p4<T, double, L, L>), dim3(g), dim3(NT), 0, s, pp, B);
+}
+
 template <typename T>
 void launch_p4(cfft_plan* p, const PipeP& pp, const PipeBufs& B, hipStream_t s) {
   if (!cubic(p)) {
@@ -850,10 +862,12 @@ void launch_p4(cfft_plan* p, const PipeP& pp, const PipeBufs& B, hipStream_t s) 
     fft_axis<T, +1>(p, static_cast<cx<T>*>(B.ch), 1, s);
     return;
   }
+  require(p->P <= kPhases, CFFT_ERR_UNSUPPORTED, "phase table larger than the kernel's copy");
   StageTimer st(p, s, CFFT_STAGE_IRECON);
   const unsigned g = (unsigned)n_planes(p);
+  const bool many = n_planes(p) >= kManyPlanes;
 #define CFFT_P4(L) \
-  case L: hipLaunchKernelGGL((k_p4<T, double, L, L>), dim3(g), dim3(p4_threads(L * L)), 0, s, pp, B); break;
+  case L: launch_p4_len<T, L>(pp, B, g, many, s); break;
   CFFT_LEN_SWITCH(p->H[1], CFFT_P4)
 #undef CFFT_P4
   launch_check<T>("k_p4");

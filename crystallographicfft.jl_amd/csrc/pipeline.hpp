@@ -474,14 +474,17 @@ __device__ __forceinline__ cx<U> csel(bool c, cx<U> a, cx<U> b) {
 // G0(q) = (1/d) sum_alpha F(q + M alpha) through the reverse-lookup table
 // (src/krfft.jl:1285-1311, src/centering_fold.jl:782-813).
 // Bound by its chain of loads (table, then the gathers of the eight aliases)
-// and by the instructions of the sum, with few workgroups: the gathers of a
-// thread's points are in flight together, lanes run along z, where neighbours
-// (h3) lie together in the spectral list, the phases come from a copy of the P
-// phases in LDS (`wl`, of kPhases entries) where it fits, and a workgroup has
-// up to 512 threads.  Ia-3d 96^3 mixed, 2 fields: 8.9 -> 6.5 us (one gather
-// after the other, 256 threads before); Im-3m 128^3 FP64, 1 field: 7.9 -> 8.6 us
-// in the trace, the backward transform 12.96 -> 12.94 us.
-constexpr int kPhases = 512;
+// and by the instructions of the sum, with few workgroups: a point's eight
+// gathers are in flight together (FP32: those of up to four of a thread's
+// points; for FP64 that takes the registers of a second workgroup, Im-3m 256^3
+// 43.7 -> 41.6 us with one point), lanes run along z, where neighbours (h3) lie
+// together in the spectral list, and the phases come from a copy of the P phases
+// in LDS (from global memory: Pmmm 192^3, 2 fields 46.6 -> 55.2 us).  P = lcm(N)
+// <= 4 H on a cubic channel grid.  Backward transforms of one field, one gather
+// after the other and 256 threads -> now: Ia-3d 96^3 12.9 -> 11.0 us mixed, 11.9
+// -> 11.5 FP64; Im-3m 128^3 14.4 -> 12.0 and 13.3 -> 13.1, 192^3 26.4 -> 20.9 and
+// 31.5 -> 24.5; two fields of Im-3m 128^3 FP64 14.9 -> 15.5 (its step 33.4 -> 30.7).
+constexpr int kPhases = 256;
 template <typename T, typename TW, int L1, int L2, int NT>
 __device__ void ph_irecon_ifft_zy(const PipeP& p, const PipeBufs& B, long item, cx<T>* lds, cx<TW>* wl) {
   constexpr int rs = L1 + 1, NP = L1 * L2, NIT = (NP + NT - 1) / NT;
@@ -504,53 +507,46 @@ __device__ void ph_irecon_ifft_zy(const PipeP& p, const PipeBufs& B, long item, 
       tb[it] = tab4[2 * (e0 + i) + 1];
     }
   }
-  constexpr int GRP = NIT % 4 == 0 ? 4 : (NIT % 3 == 0 ? 3 : (NIT % 2 == 0 ? 2 : 1));
-  auto gather = [&](const cx<TW>* w) {
+  constexpr int GRP = sizeof(T) == 8 ? 1 : (NIT % 4 == 0 ? 4 : (NIT % 3 == 0 ? 3 : (NIT % 2 == 0 ? 2 : 1)));
+  for (int i = threadIdx.x; i < p.P; i += NT) wl[i] = W[i];
+  __syncthreads();
 #pragma unroll
-    for (int i0 = 0; i0 < NIT; i0 += GRP) {
-      cx<T> f[GRP][8];
+  for (int i0 = 0; i0 < NIT; i0 += GRP) {
+    cx<T> f[GRP][8];
 #pragma unroll
-      for (int g = 0; g < GRP; ++g) {
-        const uint4 u = ta[i0 + g], v = tb[i0 + g];
-        const uint32_t ent[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+    for (int g = 0; g < GRP; ++g) {
+      const uint4 u = ta[i0 + g], v = tb[i0 + g];
+      const uint32_t ent[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
 #pragma unroll
-        for (int a = 0; a < 8; ++a) {
-          const uint32_t idx = ent[a] & 0xFFFFFu;
-          f[g][a] = Fb[idx != 0xFFFFFu ? idx : 0];
-        }
-      }
-      // keeps the loads here, together: sunk into a test of each alias they
-      // would wait for one another
-#pragma unroll
-      for (int g = 0; g < GRP; ++g) {
-#pragma unroll
-        for (int a = 0; a < 8; ++a) asm volatile("" : "+v"(f[g][a].x), "+v"(f[g][a].y));
-      }
-#pragma unroll
-      for (int g = 0; g < GRP; ++g) {
-        const int i = threadIdx.x + (i0 + g) * NT;
-        const uint4 u = ta[i0 + g], v = tb[i0 + g];
-        const uint32_t ent[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-        cx<T> acc = {T(0), T(0)};
-#pragma unroll
-        for (int a = 0; a < 8; ++a) {
-          const bool ok = (ent[a] & 0xFFFFFu) != 0xFFFFFu;
-          cx<T> fa = f[g][a];
-          if (ent[a] >> 31) fa.y = -fa.y;
-          const cx<T> prod = twmul<T, TW, -1>(fa, w[ok ? (ent[a] >> 20) & 0x7FFu : 0u]);
-          acc = cadd(acc, csel(ok, prod, {T(0), T(0)}));
-        }
-        if (i < NP)
-          lds[(i % L2) * rs + i / L2] = {(T)((TW)acc.x * p.scale_irecon), (T)((TW)acc.y * p.scale_irecon)};
+      for (int a = 0; a < 8; ++a) {
+        const uint32_t idx = ent[a] & 0xFFFFFu;
+        f[g][a] = Fb[idx != 0xFFFFFu ? idx : 0];
       }
     }
-  };
-  if (p.P <= kPhases) {
-    for (int i = threadIdx.x; i < p.P; i += NT) wl[i] = W[i];
-    __syncthreads();
-    gather(wl);
-  } else {
-    gather(W);
+    // keeps the loads here, together: sunk into a test of each alias they
+    // would wait for one another
+#pragma unroll
+    for (int g = 0; g < GRP; ++g) {
+#pragma unroll
+      for (int a = 0; a < 8; ++a) asm volatile("" : "+v"(f[g][a].x), "+v"(f[g][a].y));
+    }
+#pragma unroll
+    for (int g = 0; g < GRP; ++g) {
+      const int i = threadIdx.x + (i0 + g) * NT;
+      const uint4 u = ta[i0 + g], v = tb[i0 + g];
+      const uint32_t ent[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+      cx<T> acc = {T(0), T(0)};
+#pragma unroll
+      for (int a = 0; a < 8; ++a) {
+        const bool ok = (ent[a] & 0xFFFFFu) != 0xFFFFFu;
+        cx<T> fa = f[g][a];
+        if (ent[a] >> 31) fa.y = -fa.y;
+        const cx<T> prod = twmul<T, TW, -1>(fa, wl[ok ? (ent[a] >> 20) & 0x7FFu : 0u]);
+        acc = cadd(acc, csel(ok, prod, {T(0), T(0)}));
+      }
+      if (i < NP)
+        lds[(i % L2) * rs + i / L2] = {(T)((TW)acc.x * p.scale_irecon), (T)((TW)acc.y * p.scale_irecon)};
+    }
   }
   __syncthreads();
   lds_fft<T, TW, L2, +1, NT>(lds, L1, 1, rs);
@@ -1045,17 +1041,25 @@ __global__ void __launch_bounds__(kNT) k_p3(PipeP p, PipeBufs B) {
   ph_recon_point<T, TW>(p, B, pt, pt < (long)p.n_spec * p.batch);
 }
 
-// Threads of a P4 workgroup: the points of a plane in as few rounds as 512
-// threads allow, in whole waves.
-constexpr int p4_threads(int np) {
-  const int rounds = (np + 511) / 512;
+// Threads of a P4 workgroup: a plane's np points in as few rounds as 512
+// threads allow, in whole waves (256 threads: Im-3m 128^3, 1 field 13.1 -> 13.8 us
+// FP64, 12.0 -> 12.7 mixed; 192^3 24.5 -> 25.6, 20.9 -> 23.4).  FP64 planes that
+// fill the CUs several times over do better in smaller workgroups, more of which
+// share a CU: 384 threads at H = 64 (Im-3m 256^3, 1 and 2 fields 41.6, 76.3 ->
+// 39.5, 72.4; H = 48 is slower so, 46.6 -> 54.8 with two fields of Pmmm), and 192
+// at H = 24 from 1.5 planes per CU on (`many`: Im-3m 96^3, 6 fields 19.1 -> 17.7,
+// Pmmm 25.3 -> 22.9; below that 11.5 -> 12.2).
+constexpr int p4_threads(int np, int esz, bool many = false) {
+  const int mx = esz == 8 && many && np == 24 * 24 ? 256 : (esz == 8 && np == 64 * 64 ? 384 : 512);
+  const int rounds = (np + mx - 1) / mx;
   return ((np + rounds - 1) / rounds + 63) / 64 * 64;
 }
-template <typename T, typename TW, int L1, int L2>
-__global__ void __launch_bounds__(p4_threads(L1 * L2)) k_p4(PipeP p, PipeBufs B) {
+constexpr long kManyPlanes = 384;  // of 256 CUs
+template <typename T, typename TW, int L1, int L2, int NT = p4_threads(L1 * L2, sizeof(T))>
+__global__ void __launch_bounds__(NT) k_p4(PipeP p, PipeBufs B) {
   __shared__ cx<T> lds[L2 * (L1 + 1)];
   __shared__ cx<TW> wl[kPhases];
-  ph_irecon_ifft_zy<T, TW, L1, L2, p4_threads(L1 * L2)>(p, B, blockIdx.x, lds, wl);
+  ph_irecon_ifft_zy<T, TW, L1, L2, NT>(p, B, blockIdx.x, lds, wl);
 }
 
 template <typename T, typename TW, int L1, int L2>

@@ -36,6 +36,8 @@ LARGE = [dict(kind="steps", sg=sg, n=n, batch=b, steps=3, ds=0.01, path="qs", mi
                           (229, 256, 1), (225, 256, 1), (230, 256, 1)) for m in (False, True)]
 LARGE += [dict(kind=k, sg=sg, n=n, batch=1, mixed=m) for k in ("forward", "backward")
           for sg, n in ((229, 192), (221, 256)) for m in (False, True)]
+# both sides of the plane count from which the inverse reconstruction takes smaller workgroups
+LARGE += [dict(kind="backward", sg=229, n=96, batch=b) for b in (3, 4)]
 
 
 def _name(c):
