@@ -200,8 +200,8 @@ void build_lines(cfft_plan* p, const int (&tsel)[8][3]) {
   const int H = p->H[0], M = 2 * H, VAR = line_variant_len(H);
   const long double tp = 2.0L * 3.14159265358979323846264338327950288L;
   std::vector<double> tab((size_t)12 * VAR, 0.0);
-  std::vector<long double> cr(M), ci(M), T(H + 1), W(M), f0(M), f1r(M), f1i(M), row(H);
-  std::vector<uint64_t> by(H);
+  std::vector<long double> cr(M), ci(M), T(M), W(M), f0(M), f1r(M), f1i(M), row(H);
+  std::vector<std::pair<long double, int>> by(H);
   for (int j = 0; j < M; ++j) {
     cr[j] = cosl(tp * j / M);
     ci[j] = sinl(tp * j / M);
@@ -210,12 +210,12 @@ void build_lines(cfft_plan* p, const int (&tsel)[8][3]) {
     unsigned used = 0;
     for (int c = 0; c < p->n_ch; ++c) used |= 1u << ((axv >> (6 * c + 2 * d)) & 3);
     const long double bd = tp / p->lattice[d + 3 * d];
-    for (int q = 0; q < M; ++q) {  // (1/(2 H)) sum_a K(q + M a) [e^{-2 pi i (q + M a) t / N}]
+    for (int q = 0; q < M; ++q) {  // (1/2) sum_a K(q + M a) [e^{-2 pi i (q + M a) t / N}]
       f0[q] = f1r[q] = f1i[q] = 0.0L;
       for (int a = 0; a < 2; ++a) {
         const long h = q + (long)M * a;
         const long double kv = bd * k_centered((int)h, p->N[d]);
-        const long double kd = 0.5L * expl(-kv * kv * (long double)p->ds) / H;
+        const long double kd = 0.5L * expl(-kv * kv * (long double)p->ds);
         const long double ph = tp * (long double)((((long long)h * tsel[1 << d][d]) % p->N[d])) / p->N[d];
         f0[q] += kd;
         f1r[q] += kd * cosl(ph);
@@ -223,19 +223,19 @@ void build_lines(cfft_plan* p, const int (&tsel)[8][3]) {
       }
     }
     for (int o = 0; o < 2; ++o) {
-      if (!(used & (1u << o)) && !(used & (4u << o))) continue;
-      // A[x'][x] = T[|x' - x|] + chi W[x' + x]
+      if (!(used & (5u << o))) continue;
+      // A[x'][x] = T[x' - x + H] + chi W[x' + x]
       for (int n = 0; n < M; ++n) {
-        W[n] = 0.0L;
-        if (n <= H) T[n] = 0.0L;
-        // T is even; phase indices q n mod M of q = 2 k + o, stepped in k
-        const int step = 2 * n % M;
-        int j = o * n % M;
+        T[n] = W[n] = 0.0L;
+        // phase indices q (n - H) and q n mod M of q = 2 k + o, stepped in k
+        const int nt = (n + H) % M, st = 2 * nt % M, sw = 2 * n % M;
+        int jt = o * nt, jw = o * n;
         for (int k = 0; k < H; ++k) {
           const int q = 2 * k + o;
-          if (n <= H) T[n] += f0[q] * cr[j];
-          W[n] += f1r[q] * cr[j] - f1i[q] * ci[j];
-          j += step - (j + step >= M ? M : 0);
+          T[n] += (f0[q] * cr[jt]) / H;
+          W[n] += (f1r[q] * cr[jw] - f1i[q] * ci[jw]) / H;
+          jt += st - (jt + st >= M ? M : 0);
+          jw += sw - (jw + sw >= M ? M : 0);
         }
       }
       for (int chi = 0; chi < 2; ++chi) {
@@ -243,16 +243,13 @@ void build_lines(cfft_plan* p, const int (&tsel)[8][3]) {
         double* v = tab.data() + ((size_t)d * 4 + o + 2 * chi) * VAR;
         for (int r = 0; r < H; ++r) {
           for (int x = 0; x < H; ++x) {
-            row[x] = T[r > x ? r - x : x - r] + (chi ? -W[r + x] : W[r + x]);
-            // the magnitude's bits (positive doubles sort as integers), the position in the last ones
-            const double mag = (double)fabsl(row[x]);
-            std::memcpy(&by[x], &mag, 8);
-            by[x] = (~by[x] & ~(uint64_t)63) | (uint64_t)x;
+            row[x] = T[r - x + H] + (chi ? -W[r + x] : W[r + x]);
+            by[x] = {-fabsl(row[x]), x};
           }
-          std::sort(by.begin(), by.end());
+          std::sort(by.begin(), by.end());  // largest first, ties by position
           long double err = 0.0L;
-          for (uint64_t b : by) {
-            const int x = (int)(b & 63);
+          for (const auto& b : by) {
+            const int x = b.second;
             const double e = (double)(row[x] + err);
             err += row[x] - e;
             v[line_entry(H, r / 16, x / 4, 16 * (x % 4) + r % 16)] = e;
