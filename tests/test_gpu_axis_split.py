@@ -1,11 +1,13 @@
-"""The per-axis chain of path QS (CFFT_OPT_AXIS_SPLIT, GPU): the separable Q
-multiply applied as one 2 x 2 mixing per axis, the x mixing with the x
-transforms in the unfold/fold tile kernel and the y, z mixings in a kernel
-over single x-planes (32-point lines over eight lanes).  The same operator as
-the plane-pair chain, which the oracle pins at these sizes, up to rounding:
-sweeps agree with it to 1e-12 relative (FP64) or 2e-6 (mixed), an SCFT
-iteration's Q, F and densities to 1e-12; the option is refused where it does
-not apply."""
+"""The per-axis option of path QS (CFFT_OPT_AXIS_SPLIT, GPU).  Plans that
+accept it (a separable multiply, H = 8 to 32) run the line-matrix chain, one
+matrix per axis, with or without it: the results are the same bits.  That chain
+is compared here with an independent one on q and q+ sweeps: the plane pairs,
+which a lane split selects, where it is available (H = 16, 32), and the steps on
+the full grid elsewhere, to 1e-12 relative (FP64) or 2e-6 (mixed); an SCFT
+iteration's Q, F and densities with the plane pairs' to 1e-12.  The option is
+refused where it does not apply."""
+import functools
+
 import numpy as np
 import pytest
 
@@ -16,6 +18,7 @@ from conftest import group_setup
 pytestmark = pytest.mark.gpu
 
 
+@functools.lru_cache(maxsize=None)
 def _fields(sg, N):
     ops, ops_s, shift, R, t = group_setup(sg, N)
     Lv = O.auto_L(t)
@@ -24,12 +27,30 @@ def _fields(sg, N):
     return ops_s, wA, wB
 
 
-def _sweep(sg, N, prec, axis, ns=20, graph=1):
+@functools.lru_cache(maxsize=None)
+def _full_grid(sg, N, ns=20, f=0.3):
+    """The sweep's q and q+ from the same steps on the full grid (NumPy)."""
+    ops, ops_s, shift, R, t = group_setup(sg, N)
+    E = [np.exp(-0.5 / ns * a * O.make_symmetric(R, t, N, seed=s)) for a, s in ((2.0, 41), (-1.0, 42))]
+    K = O.fullgrid_kernel(N, 1.0 / ns, 4.0 * np.eye(3))
+    nA = int(round(f * ns))
+    out = []
+    for first, second, sw in ((E[0], E[1], nA), (E[1], E[0], ns - nA)):
+        q = np.ones(N)
+        for i in range(ns):
+            e = first if i < sw else second
+            q = e * np.fft.ifftn(K * np.fft.fftn(e * q)).real
+        out.append(O.extract_subgrid(q, O.auto_L(t)))
+    return out
+
+
+def _sweep(sg, N, prec, axis, ns=20, graph=1, lanes=0):
     import torch
     from cfft_hip.scft import PropagatorSweep
     ops_s, wA, wB = _fields(sg, N)
     sw = PropagatorSweep(N, ops_s, 4.0 * np.eye(3), 0.3, ns, prec, path=cf.PATH_QS)
     sw.plan.set_option(cf._lib.OPT_AXIS_SPLIT, axis)
+    sw.plan.set_option(cf._lib.OPT_FFT_LANES, lanes)
     sw.plan.set_option(cf._lib.OPT_GRAPH, graph)
     sw.set_fields(wA, wB)
     sw.reset()
@@ -41,20 +62,22 @@ def _sweep(sg, N, prec, axis, ns=20, graph=1):
 @pytest.mark.parametrize("sg,n", [(229, 64), (229, 128), (47, 64), (47, 128), (223, 64), (229, 32), (229, 48),
                                   (229, 96), (47, 48), (47, 32), (47, 96), (223, 96)])
 @pytest.mark.parametrize("prec,tol", [(cf.FP64, 1e-12), (cf.MIXED, 2e-6)])
-def test_axis_split_sweep_matches_plane_pairs(sg, n, prec, tol):
-    """20-step q and q+ sweep, per-axis chain against the plane-pair chain:
-    channel length H = N / 4 (8 at 32^3 to 32 at 128^3; lengths other than
-    32 on the default lane split); four channels (Im-3m, Pm-3n) or eight
-    (Pmmm: 64 tile rows, two passes of the row transforms; at 32^3 eight
-    channels of 8-row tiles fill the tile's 64 LDS rows)."""
-    print(f"axis split sg={sg} N={n} prec={prec}", flush=True)
+def test_sweep_matches_independent_chain(sg, n, prec, tol):
+    """20-step q and q+ sweep, channel length H = N / 4 (8 at 32^3 to 32 at
+    128^3), four channels (Im-3m, Pm-3n) or eight (Pmmm): the option changes no
+    bit; the plane pairs (64^3, 128^3) or the full grid give the same fields."""
+    print(f"axis option sg={sg} N={n} prec={prec}", flush=True)
     N = (n, n, n)
     a = _sweep(sg, N, prec, 0)
     b = _sweep(sg, N, prec, 1)
-    for x, y in zip(a, b):
-        err = np.max(np.abs(x - y)) / np.max(np.abs(x))
+    assert all(np.array_equal(x, y) for x, y in zip(a, b))
+    ref = _sweep(sg, N, prec, 0, lanes=2) if n in (64, 128) else _full_grid(sg, N)
+    for x, y in zip(a, ref):
+        err = np.max(np.abs(x - y)) / np.max(np.abs(y))
         print(f"  rel err {err:.2e}", flush=True)
         assert err < tol
+        if n in (64, 128) and prec == cf.FP64:
+            assert not np.array_equal(x, y)  # other kernels
 
 
 def test_axis_split_unfused_and_eager_equal_graph():
@@ -79,21 +102,23 @@ def test_axis_split_unfused_and_eager_equal_graph():
 
 
 @pytest.mark.parametrize("prec,tol", [(cf.FP64, 1e-12), (cf.MIXED, 5e-6)])
-def test_axis_split_scft_iteration(prec, tol):
+def test_scft_iterations_match_plane_pairs(prec, tol):
     """Three SCFT iterations of Im-3m 64^3 (the stored history sweep, whose
-    tile kernel writes every contour slice): Q, F and the densities with the
-    per-axis chain against the plane-pair chain."""
+    kernels write every contour slice): Q, F and the densities of the default
+    chain against the plane pairs', and with the per-axis option bit for bit."""
     from cfft_hip.scft import SCFTSolver
     N = (64, 64, 64)
     ops_s, wA, wB = _fields(229, N)
     res = []
-    for axis in (0, 1):
+    for option, value in ((cf._lib.OPT_AXIS_SPLIT, 0), (cf._lib.OPT_AXIS_SPLIT, 1), (cf._lib.OPT_FFT_LANES, 2)):
         s = SCFTSolver(N, ops_s, 4.0 * np.eye(3), 0.3, 20.0, 50, prec, path=cf.PATH_QS)
-        s.plan.set_option(cf._lib.OPT_AXIS_SPLIT, axis)
+        s.plan.set_option(option, value)
         s.set_fields(wA, wB)
         outs = [s.iterate() for _ in range(3)]
         res.append((outs, s.densities()))
-    (o0, d0), (o1, d1) = res
+    assert res[0][0] == res[1][0]
+    assert all(np.array_equal(x, y) for x, y in zip(res[0][1], res[1][1]))
+    (o0, d0), (o1, d1) = res[0], res[2]
     for a, b in zip(o0, o1):
         assert abs(a["Q"] - b["Q"]) / a["Q"] < tol
         assert abs(a["F"] - b["F"]) < tol * max(1.0, abs(a["F"]))

@@ -344,25 +344,27 @@ def test_full_size_im3m_128_properties():
     assert rel(p.diffuse(f0), p2.diffuse(f0)) < TOL64
 
 
-@pytest.mark.parametrize("path,axis", [(cf.PATH_M2, 0), (cf.PATH_QS, 0), (cf.PATH_QS, 1)])
-def test_config_pmmm_64(path, axis):
+@pytest.mark.parametrize("path,option", [(cf.PATH_M2, None), (cf.PATH_QS, None), (cf.PATH_QS, cf._lib.OPT_AXIS_SPLIT),
+                                         (cf.PATH_QS, cf._lib.OPT_FFT_LANES)])
+def test_config_pmmm_64(path, option):
     """Pmmm (#47) 64^3, cell 4.0, ds 0.01 (the reference's CPU-runnable
     configuration) at its full size: u ~ U(-1, 1) symmetrised; forward KRFFT
     at the 32768 spectral-ASU points against the full-grid FFT and the backward
-    round trip (path M2; the plane-pair chain has no backward); then 100
+    round trip (path M2; path QS has no backward); then 100
     Strang steps from q = 1 with w = 5 cos(2 pi x/a) cos(2 pi y/a)
     cos(2 pi z/a) + N(0, 0.1) symmetrised, against the same steps on the full
-    grid (NumPy FFT, K, IFFT between the two half-step factors); path QS also
-    as the per-axis chain (CFFT_OPT_AXIS_SPLIT)."""
+    grid (NumPy FFT, K, IFFT between the two half-step factors); path QS by
+    the line matrices, those with the per-axis option set (it selects no other
+    kernels), and the plane pairs (a lane split of 2)."""
     N = (64, 64, 64)
-    print(f"Pmmm 64^3 path={path} axis={axis}", flush=True)
+    print(f"Pmmm 64^3 path={path} option={option}", flush=True)
     ops, ops_s, shift, R, t = group_setup(47, N)
     Lv = O.auto_L(t)
     u = O.make_symmetric(R, t, N, seed=47, dist="uniform")
     f0 = O.extract_subgrid(u, Lv)
     plan = cf.DevicePlan(N, ops_s, DS, LAT4, path)
-    if axis:
-        plan.set_option(cf._lib.OPT_AXIS_SPLIT, 1)
+    if option is not None:
+        plan.set_option(option, 2 if option == cf._lib.OPT_FFT_LANES else 1)
     spec = O.calc_spectral_asu(R, t, N)
     assert spec.idx.shape[0] == 32768
     F = plan.forward(f0)
@@ -408,21 +410,25 @@ def test_star_coefficients(sg, N):
     assert rel(approx, O.extract_subgrid(ref, Lv)) < TOL64
 
 
-def test_mixed_chain_paired_tiles_im3m_64():
-    """Plane-pair chain at Im-3m 64^3 (H = 16: two y-blocks of 8 rows per
-    (b, z) and 32 unfold/fold workgroups per field), where the unfold/fold
-    kernel runs the two y-blocks sharing the 128-byte lines of FP32 channel
-    rows as blocks i and i + 8 of each 16.  Four Strang steps: mixed precision
-    within 2e-5 of FP64 and bit-identical across tile heights 8, 4 and 2 (a
-    different pairing each); FP64 within 1e-12 of the oracle's steps."""
+@pytest.mark.parametrize("sg", [229, 70])
+def test_mixed_chain_paired_tiles_64(sg):
+    """Plane-pair chain at 64^3 (H = 16: two y-blocks of 8 rows per (b, z) and
+    32 unfold/fold workgroups per field), where the unfold/fold kernel runs the
+    two y-blocks sharing the 128-byte lines of FP32 channel rows as blocks i and
+    i + 8 of each 16: Fddd (no line matrices) and Im-3m with the lane split that
+    selects the plane pairs.  Four Strang steps: mixed precision within 2e-5 of
+    FP64 and bit-identical across tile heights 8, 4 and 2 (a different pairing
+    each); FP64 within 1e-12 of the oracle's steps."""
     N = (64, 64, 64)
-    print("Im-3m 64^3 mixed plane-pair chain, tile heights 8/4/2", flush=True)
-    ops, ops_s, shift, R, t = group_setup(229, N)
+    print(f"sg {sg} 64^3 mixed plane-pair chain, tile heights 8/4/2", flush=True)
+    ops, ops_s, shift, R, t = group_setup(sg, N)
     Lv = O.auto_L(t)
     q = O.extract_subgrid(O.make_symmetric(R, t, N, seed=5), Lv) + 1.0
     w = 2.0 * O.extract_subgrid(O.make_symmetric(R, t, N, seed=6), Lv)
     p64 = cf.DevicePlan(N, ops_s, DS, LAT4, cf.PATH_QS)
     assert p64.H[1] == 16
+    lanes = 2 if sg == 229 else 0
+    p64.set_option(cf._lib.OPT_FFT_LANES, lanes)
     ref = p64.step(q, w, DS, nsteps=4)
     qp = O.m2q_plan(R, t, N, DS, LAT4)
     orb = O.subgrid_orbits(R, t, N, Lv)
@@ -433,6 +439,7 @@ def test_mixed_chain_paired_tiles_im3m_64():
     outs = []
     for rows in (8, 4, 2):
         p32 = cf.DevicePlan(N, ops_s, DS, LAT4, cf.PATH_QS, cf.MIXED)
+        p32.set_option(cf._lib.OPT_FFT_LANES, lanes)
         p32.set_option(cf._lib.OPT_TILE_ROWS, rows)
         outs.append(p32.step(q, w, DS, nsteps=4))
         assert rel(outs[-1], ref) < TOL32, rows

@@ -1,10 +1,14 @@
-"""Launch and radix schedules of the plane-pair chain (GPU): the plane-pair
-workgroup size (CFFT_OPT_PAIR_THREADS) leaves every result bit for bit; the
-lane split of the transforms (CFFT_OPT_FFT_LANES: R1 = 2 instead of 4, so
-16- or 8-point in-lane passes and a cross-lane radix-2 pass) reorders the
-butterflies and agrees with the default schedule, which the oracle pins at
-these sizes, to rounding; unavailable schedules are refused; the tuner
-searches both dimensions."""
+"""Launch and radix schedules of path QS (GPU): the plane-pair workgroup size
+(CFFT_OPT_PAIR_THREADS) leaves every result bit for bit, on the plans that run
+the plane pairs (Fddd: no line matrices; Im-3m with a lane split) and on those
+that run the line matrices, which ignore it; the lane split of the transforms
+(CFFT_OPT_FFT_LANES: R1 = 2 instead of 4, so 16- or 8-point in-lane passes and a
+cross-lane radix-2 pass) selects the plane pairs on Im-3m and other butterflies
+on Fddd (which round alike at H = 16), and agrees with the default chain, which the oracle pins at these
+sizes, to rounding; unavailable schedules are refused; the tuner searches both
+dimensions where they select kernels."""
+import functools
+
 import numpy as np
 import pytest
 
@@ -15,13 +19,19 @@ from conftest import group_setup
 pytestmark = pytest.mark.gpu
 
 
-def _sweep(N, prec, options, ns=20):
-    import torch
-    from cfft_hip.scft import PropagatorSweep
-    ops, ops_s, shift, R, t = group_setup(229, N)
+@functools.lru_cache(maxsize=None)
+def _fields(sg, N):
+    ops, ops_s, shift, R, t = group_setup(sg, N)
     Lv = O.auto_L(t)
     wA = 2.0 * O.extract_subgrid(O.make_symmetric(R, t, N, seed=21), Lv)
     wB = -1.0 * O.extract_subgrid(O.make_symmetric(R, t, N, seed=22), Lv)
+    return ops_s, wA, wB
+
+
+def _sweep(N, prec, options, ns=20, sg=229):
+    import torch
+    from cfft_hip.scft import PropagatorSweep
+    ops_s, wA, wB = _fields(sg, N)
     sw = PropagatorSweep(N, ops_s, 4.0 * np.eye(3), 0.3, ns, prec, path=cf.PATH_QS)
     for k, v in options.items():
         sw.plan.set_option(k, v)
@@ -32,36 +42,41 @@ def _sweep(N, prec, options, ns=20):
     return [np.asarray(x, dtype=np.float64).copy() for x in sw.fields()]
 
 
-@pytest.mark.parametrize("n", [64, 96, 128])
+@pytest.mark.parametrize("sg,n,lanes", [(70, 64, 0), (70, 96, 0), (70, 128, 0), (70, 64, 2), (229, 64, 2),
+                                        (229, 128, 2), (229, 64, 0), (229, 96, 0), (229, 128, 0)])
 @pytest.mark.parametrize("prec", [cf.FP64, cf.MIXED])
-def test_pair_threads_bit_identical(n, prec):
-    """512-thread plane-pair workgroups (H = 16, 24, 32) give the 256-thread
-    sweep bit for bit."""
-    print(f"pair threads N={n} prec={prec}", flush=True)
+def test_pair_threads_bit_identical(sg, n, lanes, prec):
+    """512-thread plane-pair workgroups (H = 16, 24, 32; the general multiply on
+    Fddd, the separable one on Im-3m with a lane split) give the 256-thread
+    sweep bit for bit; Im-3m without a lane split runs the line matrices."""
+    print(f"pair threads sg={sg} N={n} lanes={lanes} prec={prec}", flush=True)
     N = (n, n, n)
-    a = _sweep(N, prec, {})
-    b = _sweep(N, prec, {cf._lib.OPT_PAIR_THREADS: 512})
+    opt = {cf._lib.OPT_FFT_LANES: lanes}
+    a = _sweep(N, prec, opt, sg=sg)
+    b = _sweep(N, prec, {**opt, cf._lib.OPT_PAIR_THREADS: 512}, sg=sg)
     for x, y in zip(a, b):
         assert np.array_equal(x, y)
 
 
+@pytest.mark.parametrize("sg", [229, 70])
 @pytest.mark.parametrize("n", [64, 128])
 @pytest.mark.parametrize("prec,tol", [(cf.FP64, 1e-12), (cf.MIXED, 2e-6)])
-def test_lane_split_matches_default(n, prec, tol):
+def test_lane_split_matches_default(sg, n, prec, tol):
     """Lane split R1 = 2 (H = 16, 32), alone and with 512-thread plane pairs:
-    the 20-step sweep agrees with the default schedule to 1e-12 relative
-    (FP64) or 2e-6 (mixed: both schedules round to FP32 on every pass)."""
-    print(f"lane split N={n} prec={prec}", flush=True)
+    the 20-step sweep agrees with the default chain (Im-3m: line matrices,
+    Fddd: the other split) to 1e-12 relative (FP64) or 2e-6 (mixed: the plane
+    pairs round to FP32 on every pass)."""
+    print(f"lane split sg={sg} N={n} prec={prec}", flush=True)
     N = (n, n, n)
-    a = _sweep(N, prec, {})
+    a = _sweep(N, prec, {}, sg=sg)
     for opts in ({cf._lib.OPT_FFT_LANES: 2},
                  {cf._lib.OPT_FFT_LANES: 2, cf._lib.OPT_PAIR_THREADS: 512}):
-        b = _sweep(N, prec, opts)
+        b = _sweep(N, prec, opts, sg=sg)
         for x, y in zip(a, b):
             err = np.max(np.abs(x - y)) / np.max(np.abs(x))
             print(f"  {opts}: rel err {err:.2e}", flush=True)
             assert err < tol
-            if prec == cf.FP64:
+            if prec == cf.FP64 and sg == 229:
                 assert not np.array_equal(x, y)  # the option reached the kernels
 
 
