@@ -147,7 +147,7 @@ def profile_stages(sw, steps, torch):
 
 
 STRATEGY_PATH = {"m7_chain": 0, "qr_chain": 5, "qs_chain": 6, "qs_chain_eager": 6,
-                 "qs_chain_axis": 6, "qs_chain_tuned": 6}
+                 "qs_chain_tuned": 6}
 # the FETCH_SIZE / WRITE_SIZE record of each pipeline path's chain kernels
 # (eager launches and graph replays run the same kernels)
 TRAFFIC_RECORD = {0: "m7_chain", 5: "qr_chain", 6: "qs_chain"}
@@ -275,7 +275,7 @@ def scft_im3m(cf, ops_s, wA, wB, tol, max_iter):
     """Plain cold start of the Im-3m 128^3 melt (f 0.3, chiN 20, Ns 100) on the
     device, FP64: first-iteration Q, F, densities; wall time to `tol`."""
     lat = CELL * np.eye(3)
-    solver = cf.scft.SCFTSolver(N, ops_s, lat, F_A, CHIN, NS, cf.FP64, m_hist=10, axis_split=True)
+    solver = cf.scft.SCFTSolver(N, ops_s, lat, F_A, CHIN, NS, cf.FP64, m_hist=10)
     solver.set_fields(wA, wB)
     first = solver.iterate()
     phi0 = solver.densities()
@@ -523,8 +523,7 @@ def config_pmmm_64(cf, torch):
     """Pmmm (#47) 64^3, cell 4.0, ds 0.01, one field (the reference's
     CPU-runnable configuration): device-resident forward and backward KRFFT
     (us per call, 200 calls) and 100-step sweeps (field-steps/s, best of 5) on
-    each path that applies (path QS also as the per-axis chain), FP64;
-    w = 5 cos cos cos symmetrised (no noise)."""
+    each path that applies, FP64; w = 5 cos cos cos symmetrised (no noise)."""
     from cfft_hip.scft import symmetrize_subgrid
     n3 = (64, 64, 64)
     ops = cf.get_ops(47, 3, n3)
@@ -536,10 +535,8 @@ def config_pmmm_64(cf, torch):
     w = symmetrize_subgrid(5.0 * np.cos(X) * np.cos(Y) * np.cos(Z), ops_s, Lv)
     s = torch.cuda.current_stream().cuda_stream
     out = {}
-    for name, path, axis in (("m2", cf.PATH_M2, 0), ("qs_chain", cf.PATH_QS, 0), ("qs_chain_axis", cf.PATH_QS, 1)):
+    for name, path in (("m2", cf.PATH_M2), ("qs_chain", cf.PATH_QS)):
         plan = cf.DevicePlan(n3, ops_s, 0.01, lat, path)
-        if axis:  # the per-axis chain (H = 16 here)
-            plan.set_option(cf._lib.OPT_AXIS_SPLIT, 1)
         M3 = int(np.prod(plan.M))
         wd = torch.from_numpy(np.asarray(w, dtype=np.float64).ravel(order="F")).cuda()
         E = torch.exp(-wd * 0.005)
@@ -549,7 +546,7 @@ def config_pmmm_64(cf, torch):
         for what, call in (("forward", lambda: plan.forward_dev(q.data_ptr(), F.data_ptr(), s)),
                            ("backward", lambda: plan.backward_dev(F.data_ptr(), q.data_ptr(), s))):
             if what == "backward" and path == cf.PATH_QS:
-                continue  # the plane-pair chain has no F_spec backward
+                continue  # path QS has no F_spec backward
             call()
             torch.cuda.synchronize()
             t0 = time.perf_counter()
@@ -681,18 +678,16 @@ def main():
         # one is used for the timed region
         trial = {}
         sweeps = {}
-        # the plane-pair chain's schedule (tile rows, graph replay, pair
-        # workgroup size, lane split) tuned on this workload (cfft_hip.tune)
+        # path QS's schedule (graph replay; the plane pairs that a lane split
+        # selects, and their workgroup size) tuned on this workload (cfft_hip.tune)
         from cfft_hip.tune import tune_schedule
-        tuned, tuned_times = tune_schedule(N, ops_s, lat, NS, prec, 2, cf.PATH_QS, lanes=True, axis=True)
+        tuned, tuned_times = tune_schedule(N, ops_s, lat, NS, prec, 2, cf.PATH_QS, lanes=True)
         for label, path, graph in (("m7_chain", cf.PATH_AUTO, 1), ("qr_chain", cf.PATH_QR, 1),
                                    ("qs_chain", cf.PATH_QS, 1), ("qs_chain_eager", cf.PATH_QS, 0),
-                                   ("qs_chain_axis", cf.PATH_QS, 1), ("qs_chain_tuned", cf.PATH_QS, 1)):
+                                   ("qs_chain_tuned", cf.PATH_QS, 1)):
             sw = cf.scft.PropagatorSweep(N, ops_s, lat, F_A, NS, prec, path=path)
             sw.set_fields(wA, wB)
             sw.plan.set_option(cf._lib.OPT_GRAPH, graph)
-            if label == "qs_chain_axis":  # the per-axis chain of path QS
-                sw.plan.set_option(cf._lib.OPT_AXIS_SPLIT, 1)
             if label == "qs_chain_tuned":
                 for k, v in tuned.items():
                     sw.plan.set_option(k, v)

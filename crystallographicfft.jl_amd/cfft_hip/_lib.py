@@ -34,7 +34,7 @@ FP64, MIXED = 0, 1
 EXPORTED = [
     "cfft_last_error", "cfft_find_optimal_shift", "cfft_count_special_positions",
     "cfft_calc_spectral_asu", "cfft_auto_L", "cfft_select_rep_ops", "cfft_detect_centering",
-    "cfft_fill_map", "cfft_plan_create", "cfft_plan_info", "cfft_plan_tables",
+    "cfft_fill_map", "cfft_plan_create", "cfft_plan_info", "cfft_plan_line_chain", "cfft_plan_tables",
     "cfft_update_kernel", "cfft_plan_destroy", "cfft_forward", "cfft_backward",
     "cfft_forward_g0", "cfft_diffuse", "cfft_step", "cfft_sub_to_full", "cfft_full_to_sub",
     "cfft_forward_dev", "cfft_backward_dev", "cfft_diffuse_dev", "cfft_diffuse_noalloc_dev", "cfft_step_dev",
@@ -109,6 +109,7 @@ def _declare(lib):
         "cfft_fill_map": (C.c_int, [I32, PI32, PI32, I32, PI32, PI32]),
         "cfft_plan_create": (C.c_int, [PI32, PI32, I32, D, PD, I32, I32, I32, C.POINTER(P)]),
         "cfft_plan_info": (C.c_int, [P, PI32]),
+        "cfft_plan_line_chain": (C.c_int, [P, PI32]),
         "cfft_plan_tables": (C.c_int, [P, PI32, PI32, PD, PI32]),
         "cfft_update_kernel": (C.c_int, [P, D, PD]),
         "cfft_plan_destroy": (C.c_int, [P]),

@@ -261,6 +261,13 @@ class DevicePlan:
         self.ds = float(ds)
 
     @property
+    def line_chain(self):
+        """Whether diffusion, steps and sweeps run the line-matrix kernels as the options stand."""
+        on = C.c_int32()
+        L.check(L.lib().cfft_plan_line_chain(self._h, C.byref(on)))
+        return bool(on.value)
+
+    @property
     def handle(self):
         return self._h
 

@@ -171,7 +171,7 @@ class SCFTSolver:
         self.chiN = float(chiN)
         path = default_path(N, ops_shifted, lattice, precision) if path is None else path
         self.plan = DevicePlan(N, ops_shifted, 1.0 / self.ns, lattice, path, precision, batch=2)
-        if axis_split:  # CFFT_OPT_AXIS_SPLIT: checked by the plan, the kernels are the same
+        if axis_split:  # CFFT_OPT_AXIS_SPLIT: checked by the plan, selects no kernels
             self.plan.set_option(L.OPT_AXIS_SPLIT, 1)
         self.M = self.plan.M
         self.M3 = int(np.prod(self.M))

@@ -9,10 +9,12 @@ schedule computes each field with the same arithmetic), only the
 decomposition of the phase kernels and how the step sequence is launched.
 The lane split R1 x R2 of a length-H transform (in-lane R2-point passes,
 then a cross-lane radix-R1 pass) reorders the butterflies, so results move
-by rounding only; it is searched only when `lanes` is set.  CFFT_OPT_AXIS_SPLIT,
-searched when `axis` is set, no longer changes the kernels of a plan.  A timing is one
-contour sweep of `steps` Strang steps over `batch` fields with all
-interaction factors 1 (a plain multi-step sweep, the kernels of the stored
+by rounding only; it is searched only when `lanes` is set.  A plan that runs
+the line-matrix kernels ignores tile height and workgroup size: only graph
+replay is timed there and, with `lanes`, the plane pairs that a lane split
+selects instead.  CFFT_OPT_AXIS_SPLIT selects no kernels and is not timed.
+A timing is one contour sweep of `steps` Strang steps over `batch` fields with
+all interaction factors 1 (a plain multi-step sweep, the kernels of the stored
 sweeps apart from the q store), after one untimed sweep that captures the
 graph; the best of `reps` sweeps counts.  The grid of tile heights x graph
 replay is timed in full, then each further dimension from the best so far.
@@ -36,26 +38,28 @@ def schedule_candidates(H1):
     return [{L.OPT_TILE_ROWS: r, L.OPT_GRAPH: g} for r in rows for g in (1, 0)]
 
 
-def extra_dimensions(plan, lanes, axis=False):
-    """Further schedule dimensions of a plan on path QS: with `axis`, the
-    per-axis option (H = 8, 12, 16, 24, 32; plans without the separable
-    multiply refuse it); the plane-pair workgroup size (512 threads
-    for H = 16, 24, 32) and, with `lanes`, the lane split R1 = 2 of the
-    transforms (H = 16, 32)."""
+def plan_candidates(plan):
+    """The grid of schedules that select kernels of `plan`."""
+    if plan.line_chain:
+        return [{L.OPT_TILE_ROWS: 0, L.OPT_GRAPH: g} for g in (1, 0)]
+    return schedule_candidates(plan.H[1])
+
+
+def extra_dimensions(plan, lanes):
+    """Further schedule dimensions of a plan on path QS: the plane-pair
+    workgroup size (512 threads for H = 16, 24, 32) and, with `lanes`, the lane
+    split R1 = 2 of the transforms (H = 16, 32), which comes first on a plan of
+    line matrices, where the workgroup size has no meaning without it."""
     out = []
     if plan.path == L.PATH_QS:
-        if axis and plan.H[0] in (8, 12, 16, 24, 32):
-            out.append((L.OPT_AXIS_SPLIT, 1))
-        if plan.H[1] in (16, 24, 32):
-            out.append((L.OPT_PAIR_THREADS, 512))
-        if lanes and plan.H[0] in (16, 32):
-            out.append((L.OPT_FFT_LANES, 2))
+        split = [(L.OPT_FFT_LANES, 2)] if lanes and plan.H[0] in (16, 32) else []
+        pair = [(L.OPT_PAIR_THREADS, 512)] if plan.H[1] in (16, 24, 32) else []
+        out = (split + pair if split else []) if plan.line_chain else pair + split
     return out
 
 
 def _label(opt):
     return (f"rows{opt[L.OPT_TILE_ROWS]}_graph{opt[L.OPT_GRAPH]}"
-            + ("_axis" if opt.get(L.OPT_AXIS_SPLIT) else "")
             + (f"_pt{opt[L.OPT_PAIR_THREADS]}" if opt.get(L.OPT_PAIR_THREADS) else "")
             + (f"_lanes{opt[L.OPT_FFT_LANES]}" if opt.get(L.OPT_FFT_LANES) else ""))
 
@@ -71,10 +75,8 @@ def tune_schedule(N, ops_shifted, lattice, ns, precision, batch, path, steps=Non
                   axis=False):
     """(best options, {label: microseconds per step}) for a plan of `batch`
     fields with ds = 1/ns; options are {OPT_TILE_ROWS: r, OPT_GRAPH: g,
-    OPT_PAIR_THREADS: t, OPT_FFT_LANES: l} (the last two 0 = default), plus
-    OPT_AXIS_SPLIT with `axis`.  A candidate the plan refuses (the per-axis
-    chain without the separable multiply, or with the R1 = 2 lane split) is
-    skipped."""
+    OPT_PAIR_THREADS: t, OPT_FFT_LANES: l} (0 = default, also the tile height
+    of a plan of line matrices), plus OPT_AXIS_SPLIT: 0 with `axis`."""
     import torch
     key = _key(N, ops_shifted, lattice, ns, precision, batch, path) + (bool(lanes), bool(axis))
     if key in _CACHE:
@@ -89,8 +91,6 @@ def tune_schedule(N, ops_shifted, lattice, ns, precision, batch, path, steps=Non
     times = {}
 
     def timed(opt):
-        # the per-axis chain first: it excludes the R1 = 2 lane split
-        plan.set_option(L.OPT_AXIS_SPLIT, opt.get(L.OPT_AXIS_SPLIT, 0))
         for k, v in opt.items():
             plan.set_option(k, v)
         plan.step_dev(q.data_ptr(), E.data_ptr(), steps, s)  # captures the graph when enabled
@@ -106,7 +106,7 @@ def tune_schedule(N, ops_shifted, lattice, ns, precision, batch, path, steps=Non
         return t
 
     best, best_t = None, None
-    for opt in schedule_candidates(plan.H[1]):
+    for opt in plan_candidates(plan):
         opt = dict(opt)
         opt.update({L.OPT_PAIR_THREADS: 0, L.OPT_FFT_LANES: 0})
         if axis:
@@ -114,29 +114,15 @@ def tune_schedule(N, ops_shifted, lattice, ns, precision, batch, path, steps=Non
         t = timed(opt)
         if best_t is None or t < best_t:
             best, best_t = opt, t
-
-    def trial(opt):
-        nonlocal best, best_t
-        try:
-            t = timed(opt)
-        except L.CFFTError as e:
-            if e.code != L.CFFT_ERR_UNSUPPORTED:
-                raise
-            return False
+    lines = plan.line_chain
+    opt = dict(best)
+    for k, v in extra_dimensions(plan, lanes):
+        # on a plan of line matrices the pairs' workgroup size is tried with the
+        # lane split that selects them, otherwise each dimension from the best
+        opt = {**(opt if lines else best), k: v}
+        t = timed(opt)
         if t < best_t:
             best, best_t = opt, t
-        return True
-
-    grid_best = dict(best)
-    for k, v in extra_dimensions(plan, lanes, axis):
-        opt = dict(best)
-        opt[k] = v
-        if trial(opt) and k == L.OPT_AXIS_SPLIT:
-            # the per-axis chain's kernels cut the tiles differently: every
-            # tile height with the best graph setting
-            for r in sorted({c[L.OPT_TILE_ROWS] for c in schedule_candidates(plan.H[1])}):
-                if r != grid_best[L.OPT_TILE_ROWS]:
-                    trial({**grid_best, L.OPT_TILE_ROWS: r, L.OPT_AXIS_SPLIT: 1})
     del plan
     _CACHE[key] = (best, times)
     return best, times

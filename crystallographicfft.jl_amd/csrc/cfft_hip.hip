@@ -68,7 +68,7 @@ struct cfft_plan {
   int arith32 = 0;     // mixed precision on path QS: FP32 twiddle and fold-factor arithmetic (option)
   int lanes = 0;       // path QS: lane split of the plane-pair and tile transforms (0: the default)
   int pair_threads = 0;  // path QS: threads per plane-pair workgroup (0: 256)
-  int axis_split = 0;    // path QS: the per-axis chain (x mixing in the tile kernel, single planes)
+  int axis_split = 0;    // path QS: the per-axis option, which selects no kernels (ensembles refuse it)
   hipStream_t cap_stream = nullptr;  // capture stream of the chains
   struct Cached {
     std::string key;
@@ -1672,6 +1672,14 @@ int cfft_plan_info(const cfft_plan* p, int32_t* info) {
                      p->cent, p->d,    p->path, p->prec, p->batch, p->H[0], p->H[1], p->H[2],
                      (int32_t)p->n_rep, (int32_t)p->n_alive};
     std::memcpy(info, v, sizeof(v));
+  });
+}
+
+int cfft_plan_line_chain(const cfft_plan* p, int32_t* on) {
+  return guarded([&] {
+    check_plan(p);
+    require(on != nullptr, CFFT_ERR_INVALID, "null argument");
+    *on = use_lines(p) ? 1 : 0;
   });
 }
 

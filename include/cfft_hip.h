@@ -134,6 +134,9 @@ int cfft_plan_create(const int32_t* N, const int32_t* ops, int32_t nops, double 
  * d, path, precision, batch, H0, H1, H2, n_rep (path QR orbit representatives,
  * else 0), n_alive (channel elements per field)}. */
 int cfft_plan_info(const cfft_plan* plan, int32_t* info);
+/* *on = 1 if the plan's diffusion, steps and sweeps run the line-matrix
+ * kernels as its options stand, else 0. */
+int cfft_plan_line_chain(const cfft_plan* plan, int32_t* on);
 
 /* Spectral-ASU points of the plan: idx_out (n_spec x 3), mult_out (n_spec);
  * K_out (n_spec) = diffusion kernel; rep_out (d) = representative op indices.

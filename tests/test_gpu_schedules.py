@@ -115,8 +115,8 @@ def test_schedule_options_refused():
 
 
 def test_tuner_searches_radix_schedule():
-    """tune_schedule(lanes=True) on Im-3m 64^3 (H = 16) times the tile/graph
-    grid, then 512-thread pairs and the R1 = 2 lane split from the best; the
+    """tune_schedule(lanes=True) on Im-3m 64^3 (H = 16) times graph replay, then
+    the plane pairs of the R1 = 2 lane split, and those with 512 threads; the
     returned options name all four settings."""
     from cfft_hip.tune import tune_schedule
     N = (64, 64, 64)

@@ -1,5 +1,5 @@
-"""The 32-point line transform over eight lanes of four values (the per-axis
-chain's line transforms, csrc/fft.hpp fft32_l8_lds) restated in NumPy: the
+"""A 32-point line transform over eight lanes of four values, restated in NumPy
+(no kernel uses this split since path QS applies its axes as matrices): the
 in-lane 4-point DFTs of x[r + 8 m], the twiddles w32^(r k), and per lane
 r = 2 k + h the parity half of the 8-point DFT across the lanes,
 X[k + 4 (h + 2 j)] = sum_s w8^(s h) w4^(s j) (y_s + (-1)^h y_{s+4}),
